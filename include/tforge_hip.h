@@ -38,6 +38,9 @@ extern "C" {
 #define TF_E_BLAS -6     /* vendor BLAS baseline unavailable or failed        */
 
 #define TF_FAMILY_DIRECT 0      /* tile-k=0: one FMA chain per output          */
+/* (A TF_FAMILY_DIRECT launch reports the options' own geometry.  On 16-byte
+ * aligned buffers its chains run on the matrix cores, in workgroups the library
+ * sizes to the problem; the result is the same bits.) */
 #define TF_FAMILY_STAGED 1      /* tile-k>0: LDS-staged FP32 MFMA              */
 #define TF_FAMILY_ELEMENTWISE 2 /* programs without a matmul                   */
 #define TF_FAMILY_WAVEK 4       /* tile-k>0 with wave-split-k: the waves of a

@@ -6,7 +6,10 @@
 // TM x TN sub-tile of its block tile and runs the K loop from +0.0 with one
 // fused multiply-add per k, in sequential k order, then the fused epilogue.
 // That arithmetic is bit-identical to the reference's naive kernel
-// (docs/numerics.md:53), any shape is accepted and edges are masked.
+// (docs/numerics.md:53), any shape is accepted and edges are masked.  Where
+// every buffer is 16-byte aligned the runtime runs the same chains on the matrix
+// cores instead (staged_gemm.hpp, sequential k; the same bits); this kernel
+// serves the rest: unaligned buffers, and ragged matrices of 2^31 elements.
 //
 // Element-op kernels: programs with no matmul (tforge.bias_add / relu / add
 // alone, or chains of them) run one thread per TM x TN elements with the same

@@ -194,6 +194,17 @@ def name(c):
             + ("_masked" if mk else ""))
 
 
+# Sequential-k instantiations: the matrix-core form of the direct kernel (tile-k
+# = 0), chosen by the runtime from the problem's size (seq_entry in
+# runtime.hip), not by an option string; each with a masked twin.
+SEQ_CONFIGS = [(32, 32, 2, 2, 32), (32, 32, 2, 2, 64), (64, 64, 4, 4, 16), (128, 128, 8, 8, 16)]
+
+
+def seq_name(c):
+    bm, bn, tm, tn, bk, mk = c
+    return f"tf_seq_b{bm}x{bn}_t{tm}x{tn}_k{bk}" + ("_masked" if mk else "")
+
+
 def main(shards=16):
     gen = HERE / "_gen"
     gen.mkdir(exist_ok=True)
@@ -238,6 +249,25 @@ def main(shards=16):
     lines += ["#endif", "", "}  // namespace tfk", ""]
     text = "\n".join(lines)
     p = gen / "wavek.hip"
+    if not p.exists() or p.read_text() != text:
+        p.write_text(text)
+    seq = [c + (mk,) for c in SEQ_CONFIGS for mk in (0, 1)]
+    lines = ['#include "../staged_gemm.hpp"', "", "namespace tfk {", "",
+             "#ifndef __HIP_DEVICE_COMPILE__  // host table", "extern const KernelEntry kSeqEntries[] = {"]
+    for c in seq:
+        bm, bn, tm, tn, bk, mk = c
+        t = f"{bm}, {bn}, {tm}, {tn}, {bk}, 1, 1"
+        lines.append(f"    KernelEntry{{FAM_DIRECT, {t}, {mk}, \"{seq_name(c)}\",")
+        lines.append(f"                reinterpret_cast<const void *>(&staged_gemm_kernel<{t}, {mk}, 1>),")
+        lines.append(f"                &launch_staged<{t}, {mk}, 1>, nullptr, StagedGemm<{t}, 1>::LDS_BYTES}},")
+    lines += ["};", f"extern const int kSeqCount = {len(seq)};", "#else",
+              "// Device pass: instantiate the kernels the host table names."]
+    for bm, bn, tm, tn, bk, mk in seq:
+        lines.append(f"template __global__ void staged_gemm_kernel<{bm}, {bn}, {tm}, {tn}, {bk}, 1, 1, {mk}, 1>(const float *, "
+                     "const float *, long, long, int, int, int, int, int, int, GemmParams);")
+    lines += ["#endif", "", "}  // namespace tfk", ""]
+    text = "\n".join(lines)
+    p = gen / "seq.hip"
     if not p.exists() or p.read_text() != text:
         p.write_text(text)
     reg = ['#include <vector>', '', '#include "../tf_kernels.h"', '', 'namespace tfk {', '',

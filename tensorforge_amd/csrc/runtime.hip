@@ -116,9 +116,56 @@ void staged_wave_layout(long bm, long bn, long tm, long tn, long &ktm, long &ktn
 struct Launch {
   const tfk::KernelEntry *entry = nullptr;
   dim3 grid, block;
+  // Direct GEMMs: the matrix-core form of the same arithmetic that runs
+  // instead wherever every buffer is 16-byte aligned (seq_entry), with its own
+  // geometry; null where the problem has none.
+  const tfk::KernelEntry *seq = nullptr;
+  dim3 seq_grid, seq_block;
 };
 
 long ceil_div(long a, long b) { return (a + b - 1) / b; }
+
+// The matrix-core kernel that runs a direct GEMM (tile-k = 0) of this size, or
+// null where only the one-thread-per-tile kernel can.  A rule on sizes alone:
+// the results are the same bits whichever tile runs.
+//
+// Predicted time = start + rounds * K * cost, rounds = ceil(tiles / 256) (one
+// workgroup per CU each); the tile with the least runs.  Measured on MI355X:
+// cost 5.6-6.0 ns per k for 32x32 tiles, 15.1-16.4 for 64x64, 59-60 for 128x128
+// (masked twins about 1/12 more), start 2.7, 3.4 and 5.7 us.  Both sides of
+// the lines (us, back to back): 32 / 64 at 700^3 11.2 / 16.1, 900^3 22.0 / 20.1,
+// 1100^3 38.5 / 38.8, 64x4096x4096 24.0 / 71.9; 64 / 128 at 1800x1800x500
+// 37.5 / 42.7, 2048^3 126.1 / 125.3, 4096x4096x1024 256.8 / 247.4,
+// 4095x4097x1023 283.0 / 324.6.  With the small tile a K of 2048 or more takes
+// tile-k 64: one workgroup per CU streams its operands, and twice the loads in
+// flight carry it (64x4096x4096 33.0 -> 24.0, 64x2048x2048 12.7 -> 12.1); below
+// that tile-k 32 starts sooner and pads less (700^3 11.2 against 12.2).
+const tfk::KernelEntry *seq_entry(long M, long N, long K) {
+  struct Tile {
+    long edge, cost, start;  // tenths of ns
+  };
+  constexpr Tile kTiles[] = {{32, 57, 27000}, {64, 155, 34000}, {128, 590, 57000}};
+  constexpr long kCus = 256;
+  auto small_k = [&] { return K >= 2048 ? 64 : 32; };
+  auto ragged = [&](long edge) { return M % edge || N % edge || K % (edge == 32 ? small_k() : 16) ? 1 : 0; };
+  const Tile *best = nullptr;
+  double best_time = 0;
+  for (const Tile &t : kTiles) {
+    const double rounds = (double)ceil_div(ceil_div(M, t.edge) * ceil_div(N, t.edge), kCus);
+    const double time = t.start + rounds * K * (t.cost + (ragged(t.edge) ? t.cost / 12 : 0));
+    if (!best || time < best_time) best = &t, best_time = time;
+  }
+  for (int i = 0; i < tfk::kSeqCount; ++i) {
+    const tfk::KernelEntry &e = tfk::kSeqEntries[i];
+    if (e.bm != best->edge || (e.bm == 32 && e.bk != small_k()) || e.masked != ragged(e.bm)) continue;
+    // The kernels number the tiles in 32 bits; masked twins index A and B with
+    // 32-bit offsets (tiles may run one block past the edges).
+    if (ceil_div(M, e.bm) * ceil_div(N, e.bn) >= (1L << 31)) return nullptr;
+    if (e.masked && ((M + 256) * K >= (1L << 31) || (K + 64) * (N + 256) >= (1L << 31))) return nullptr;
+    return &e;
+  }
+  return nullptr;
+}
 
 }  // namespace
 
@@ -233,6 +280,13 @@ int select_launches(tf_kernel *k) {
                                                     " threads per block exceeds 1024"));
     L.block = dim3((unsigned)tx, (unsigned)ty, 1);
     L.grid = dim3((unsigned)std::max(1L, ceil_div(st.N, o.bn)), (unsigned)std::max(1L, ceil_div(st.M, o.bm)), 1);
+    if (gemm && !staged && st.M > 0 && st.N > 0) {
+      L.seq = seq_entry(st.M, st.N, st.K);
+      if (L.seq) {
+        L.seq_block = dim3((unsigned)(L.seq->bn / L.seq->tn), (unsigned)(L.seq->bm / L.seq->tm), 1);
+        L.seq_grid = dim3((unsigned)ceil_div(st.N, L.seq->bn), (unsigned)ceil_div(st.M, L.seq->bm), 1);
+      }
+    }
     // split-k splits the K loop of GEMM stages; the element-op launches of an
     // unfused program run as they are.  Without tile-k it is an error.
     if (o.split_k > 1 && (gemm || o.tile_k == 0)) {
@@ -273,13 +327,18 @@ int launch_stage(const tf_kernel *k, size_t s, void *const *ptrs, void *ws, hipS
   if (st.M == 0 || st.N == 0) return TF_OK;
   // 128-bit accesses need 16-byte aligned buffers (the reference's ABI
   // guarantees 256-byte alignment: docs/stage8.md:34).
-  if (L.entry->family == tfk::FAM_STAGED || L.entry->family == tfk::FAM_WAVEK) {
+  bool use_seq = L.seq != nullptr;
+  if (use_seq || L.entry->family == tfk::FAM_STAGED || L.entry->family == tfk::FAM_WAVEK) {
     std::vector<int> ids = {st.a, st.b, st.out};
     for (const tff::EpiOp &e : st.epi)
       if (e.buf >= 0) ids.push_back(e.buf);
     for (int id : ids)
-      if (reinterpret_cast<uintptr_t>(ptrs[id]) % 16 != 0)
-        return fail(TF_E_ARG, "buffer " + std::to_string(id) + " is not 16-byte aligned");
+      if (reinterpret_cast<uintptr_t>(ptrs[id]) % 16 != 0) {
+        // The direct kernel takes any alignment.
+        if (!use_seq) return fail(TF_E_ARG, "buffer " + std::to_string(id) + " is not 16-byte aligned");
+        use_seq = false;
+        break;
+      }
   }
   hipError_t err;
   if (st.kind == tff::STAGE_GEMM) {
@@ -301,7 +360,7 @@ int launch_stage(const tf_kernel *k, size_t s, void *const *ptrs, void *ws, hipS
       p.ws_ld = (long)L.grid.x * L.entry->bn;
       p.ws_slice = p.ws_ld * L.grid.y * L.entry->bm;
     }
-    err = L.entry->gemm(p, L.grid, L.block, stream);
+    err = use_seq ? L.seq->gemm(p, L.seq_grid, L.seq_block, stream) : L.entry->gemm(p, L.grid, L.block, stream);
     if (err == hipSuccess && p.splits > 1) {
       tfk::ReduceParams r{};
       r.ws = p.ws;

@@ -20,6 +20,18 @@
 //    one column.  The sum order differs from the reference's sequential k;
 //    parity is the reference's own FP64 error bound, which holds for any
 //    order (python/tforge_cpu.py:263-271).
+//  * Sequential k (SEQ = 1, the matrix-core form of the direct kernel).  On
+//    gfx950 the FP32 MFMAs accumulate one fused multiply-add per k, lane group
+//    0's k first (bit for bit against fmaf over random, wide-exponent,
+//    denormal and infinite operands), so a chunk whose step s and lane group
+//    g take k = KC*kc + (64/MB)*s + g computes exactly the direct kernel's
+//    chain.  A is stored to LDS with the k of a chunk in (g, s) order, so its
+//    fragments stay one ds_read_b128; B fragments read rows (64/MB)*s + g.
+//    The K tail of A is padded with -0.0: -0.0 * +0.0 = -0.0 leaves every
+//    accumulator as it is, a -0.0 included (+0.0 would make it +0.0).  Bound
+//    by the same matrix pipes as the staged kernels; back to back, one thread
+//    per output -> this: 256x256x128 15.2 -> 3.5 us, 777x1111x333 132 -> 11.4,
+//    1000^3 376-471 -> 21.3, 2048^3 3763 -> 125.3 (137 TFLOP/s).
 //  * Staging (promote=1).  A tile [BM][BK+4 or +8] and B tile [BK][BN+8 or +4] in LDS,
 //    double-buffered, one barrier per slab.  Two register staging sets where
 //    a thread stages few vectors: the global loads of slab t+3 are issued in
@@ -61,6 +73,7 @@
 
 namespace tfk {
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // One MFMA on an MB x MB block: acc += src0 (4 x MB, from B) ^T-contracted with
@@ -120,7 +133,7 @@ __device__ __forceinline__ VT buffer_load_vt(__amdgpu_buffer_rsrc_t rs, int byte
 __device__ __forceinline__ void put(float &v, int, float x) { v = x; }
 __device__ __forceinline__ void put(f32x4 &v, int e, float x) { v[e] = x; }
 
-template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC>
+template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC, int SEQ = 0>
 struct StagedGemm {
   static constexpr int NT = (BM / TM) * (BN / TN);
   static constexpr int WTM = 8 * TM, WTN = 8 * TN;
@@ -135,7 +148,12 @@ struct StagedGemm {
   static constexpr int LDA = BK + ((WTM % 32 == 0 && WTN % 32 == 0) ? 4 : 8);
   // LDS B row stride: the 64 / MB lane groups read rows 4 apart; +8 (MB = 32)
   // or +4 (MB = 16) puts them in disjoint banks.
-  static constexpr int LDB = BN + (MB == 32 ? 8 : 4);
+  // SEQ: the lane groups read adjacent rows instead; a stride of 32 (MB = 32)
+  // or 16 (MB = 16) mod 64 floats puts those in disjoint banks.
+  static constexpr int LDB = SEQ ? (MB == 32 ? BN + (BN % 64 == 0 ? 32 : 0) : BN + 16) : BN + (MB == 32 ? 8 : 4);
+  // Row of the B slab that lane group g reads at step s of chunk kc:
+  // kc * KC + g * B_ROW_G + s * B_ROW_S (see "K order").
+  static constexpr int B_ROW_G = SEQ ? 1 : 4, B_ROW_S = SEQ ? 64 / MB : 1;
   static constexpr int A_ELEMS = BM * LDA, B_ELEMS = BK * LDB;
   // Two A and B tile buffers, plus the tile's BN bias values.
   static constexpr int LDS_BYTES = PROMOTE ? 2 * (A_ELEMS + B_ELEMS) * 4 + BN * 4 : 0;
@@ -172,6 +190,18 @@ struct StagedGemm {
     }
   }
 
+  // LDS position, in its row, of element e of the A staging vector at column
+  // c.  Each lane group reads 4 consecutive positions, 4 * g + s of a chunk.
+  // SEQ: position 4 * g + s of a chunk holds k = s * (64 / MB) + g, the order in
+  // which the MFMA's lane groups contract it.
+  static __host__ __device__ __forceinline__ constexpr int a_pos(int c, int e) {
+    if constexpr (!SEQ) return c + e;
+    constexpr int G = 64 / MB;
+    const int kk = c % KC + e;
+    return c - c % KC + 4 * (kk % G) + kk / G;
+  }
+
+  static_assert(!SEQ || (PROMOTE && VEC), "sequential-k instantiations stage through LDS with 128-bit loads");
   static_assert(BM % TM == 0 && BN % TN == 0, "block tile must be a multiple of the thread tile");
   static_assert(NWM * NWN * 64 == NT, "waves must tile the block");
   static_assert(WTM % 16 == 0 && WTN % 16 == 0, "wave tile must be made of 16x16 or 32x32 MFMA blocks");
@@ -187,7 +217,7 @@ struct StagedGemm {
 // by-value struct is read from the kernel-argument segment (a ~1.5k-cycle
 // round trip measured at the start of every wave).  gx, gy = gridDim.x, .y;
 // flags = swizzle | splits << 8.
-template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC, int MASK>
+template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC, int MASK, int SEQ = 0>
 __global__ void __launch_bounds__((BM / TM) * (BN / TN))
 staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int pK, int gx, int gy, int flags, int pM,
                    int pN, GemmParams p) {
@@ -200,7 +230,7 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
   p.N = pN;
   p.swizzle = flags & 255;
   p.splits = flags >> 8;
-  using G = StagedGemm<BM, BN, TM, TN, BK, PROMOTE, VEC>;
+  using G = StagedGemm<BM, BN, TM, TN, BK, PROMOTE, VEC, SEQ>;
   constexpr int NT = G::NT, WTM = G::WTM, WTN = G::WTN, NWN = G::NWN, FM = G::FM, FN = G::FN;
   constexpr int LDA = G::LDA, LDB = G::LDB, VW = G::VW, MB = G::MB, KC = G::KC;
   using AccT = AccOf<MB>;
@@ -407,6 +437,19 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
         }
       }
     };
+    auto store_a = [&](float *row, int c, const VT &v) __attribute__((always_inline)) {
+      if constexpr (!SEQ) {
+        *reinterpret_cast<VT *>(row + c) = v;
+      } else if constexpr (MB == 32) {
+        float *dst = row + G::a_pos(c, 0);
+        *reinterpret_cast<f32x2 *>(dst) = f32x2{v.x, v.z};
+        *reinterpret_cast<f32x2 *>(dst + 4) = f32x2{v.y, v.w};
+      } else {
+        float *dst = row + G::a_pos(c, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dst[4 * e] = v[e];
+      }
+    };
     auto store_slab = [&](auto sc, auto gm, int buf, int k0) __attribute__((always_inline)) {
       constexpr int set = decltype(sc)::value;
       if (MASK && decltype(gm)::value == 1 && guarded(k0)) {
@@ -414,7 +457,7 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
         for (int it = 0; it < G::A_PER; ++it)
 #pragma unroll
           for (int e = 0; e < VW; ++e)
-            if (!a_in(tid + it * NT, k0, e)) put(ra[set][it], e, 0.0f);
+            if (!a_in(tid + it * NT, k0, e)) put(ra[set][it], e, SEQ ? -0.0f : 0.0f);
 #pragma unroll
         for (int it = 0; it < G::B_PER; ++it)
 #pragma unroll
@@ -427,7 +470,7 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
         if (G::A_VECS % NT == 0 || q < G::A_VECS) {
           int r, c;
           G::a_item(q, r, c);
-          *reinterpret_cast<VT *>(&As[buf][r * LDA + c]) = ra[set][it];
+          store_a(&As[buf][r * LDA], c, ra[set][it]);
         }
       }
 #pragma unroll
@@ -508,7 +551,7 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
         if (G::A_VECS % NT == 0 || q < G::A_VECS) {
           int r, c;
           G::a_item(q, r, c);
-          *reinterpret_cast<VT *>(&As[buf][r * LDA + c]) = ra[set][it];
+          store_a(&As[buf][r * LDA], c, ra[set][it]);
         }
       } else {
         const int q = tid + (it - G::A_PER) * NT;
@@ -520,7 +563,7 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     };
     auto load_frags = [&](int buf, int kc, int slot) __attribute__((always_inline)) {
       const float *as = As[buf] + (wm * WTM + lr) * LDA + 4 * lg + kc * KC;
-      const float *bs = Bs[buf] + (4 * lg + kc * KC) * LDB + wn * WTN + lr;
+      const float *bs = Bs[buf] + (G::B_ROW_G * lg + kc * KC) * LDB + wn * WTN + lr;
 #pragma unroll
       for (int i = 0; i < FM; ++i) {
         const float *src = as + i * MB * LDA;
@@ -536,7 +579,7 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
 #pragma unroll
       for (int j = 0; j < FN; ++j)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) bf[slot][j][s] = bs[s * LDB + j * MB];
+        for (int s = 0; s < 4; ++s) bf[slot][j][s] = bs[s * G::B_ROW_S * LDB + j * MB];
     };
     // Slab 0's loads go out first: the bias test reads the epilogue fields
     // from the kernel-argument segment, and its wait would delay them.
@@ -820,10 +863,10 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
   }
 }
 
-template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC, int MASK>
+template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC, int MASK, int SEQ = 0>
 hipError_t launch_staged(const GemmParams &p, dim3 grid, dim3 block, hipStream_t stream) {
   if (block.x != BN / TN || block.y != BM / TM || block.z != 1) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((staged_gemm_kernel<BM, BN, TM, TN, BK, PROMOTE, VEC, MASK>), grid, block, 0, stream, p.A, p.B,
+  hipLaunchKernelGGL((staged_gemm_kernel<BM, BN, TM, TN, BK, PROMOTE, VEC, MASK, SEQ>), grid, block, 0, stream, p.A, p.B,
                      p.lda, p.ldb, p.K, (int)grid.x, (int)grid.y, p.swizzle | (p.splits << 8), p.M, p.N, p);
   return hipGetLastError();
 }

@@ -86,6 +86,11 @@ struct KernelEntry {
 // The split-K reduction (direct_kernels.hip); ws and C 16-byte aligned.
 hipError_t launch_splitk_reduce(const ReduceParams &p, hipStream_t stream);
 
+// The sequential-k staged instantiations (generated _gen/seq.hip): the
+// matrix-core form of the direct kernel, each followed by its masked twin.
+extern const KernelEntry kSeqEntries[];
+extern const int kSeqCount;
+
 // Registry (defined in the generated registry translation unit).
 const KernelEntry *registry_begin();
 const KernelEntry *registry_end();
