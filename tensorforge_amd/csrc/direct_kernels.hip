@@ -12,12 +12,13 @@
 // serves the rest: unaligned buffers, and ragged matrices of 2^31 elements.
 //
 // Element-op kernels: programs with no matmul (tforge.bias_add / relu / add
-// alone, or chains of them) run one thread per TM x TN elements with the same
-// launch geometry, one IEEE operation per op, so results are bit-exact against
-// NumPy float32 (python/tforge_gpu.py:116-126).
+// alone, or chains of them) run one IEEE operation per op, so results are
+// bit-exact against NumPy float32 (python/tforge_gpu.py:116-126).
 //
 // Split-K reduction: the second launch of a staged matmul compiled with
 // split-k=S (a backend option): C = epi(slice 0 + ... + slice S-1).
+#include <algorithm>
+
 #include "epilogue.hpp"
 
 namespace tfk {
@@ -53,49 +54,12 @@ __global__ void direct_gemm_kernel(GemmParams p) {
     }
 }
 
+// Element ops on buffers that are not 16-byte aligned: the options' own
+// geometry, one element at a time.
 template <int TM, int TN>
 __global__ void elementwise_kernel(EltParams p) {
   const long m_base = ((long)blockIdx.y * blockDim.y + threadIdx.y) * TM;
   const long n_base = ((long)blockIdx.x * blockDim.x + threadIdx.x) * TN;
-  if constexpr (TN % 4 == 0) {
-    // Thread tiles 4k wide on aligned rows: 128-bit loads and stores, so a
-    // wave moves 64 x TN x 4 contiguous bytes per row.  Same IEEE ops.  Every
-    // byte is read or written once, so the accesses are non-temporal (MI355X:
-    // 6.80 against 6.38 TB/s for relu at 16384^2 with cached accesses).
-    if (p.vec_ok && n_base + TN <= p.N) {
-      // All loads first (rows past M read row M-1 and are not stored), so
-      // they are in flight together; then the ops and the stores.  A chain
-      // that starts with bias_add loads its bias here too (cached: every row
-      // reads it), rather than behind the epilogue's per-op branch, where
-      // each thread would wait for X before asking for the bias.
-      const bool pre_bias = p.epi.nops > 0 && p.epi.kind[0] == EPI_BIAS;
-      f32x4 bv[TN / 4];
-#pragma unroll
-      for (int j = 0; j < TN / 4; ++j)
-        bv[j] = pre_bias ? *reinterpret_cast<const f32x4 *>(p.epi.ptr[0] + n_base + 4 * j) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      f32x4 x[TM][TN / 4];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const long m = min(m_base + i, (long)p.M - 1);
-#pragma unroll
-        for (int j = 0; j < TN / 4; ++j)
-          x[i][j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(p.X + m * p.ldx + n_base + 4 * j));
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const long m = m_base + i;
-        if (m >= p.M) break;
-#pragma unroll
-        for (int j = 0; j < TN / 4; ++j) {
-          const int n = (int)n_base + 4 * j;
-          const f32x4 v = pre_bias ? apply_epi4<true>(x[i][j] + bv[j], p.epi, m, n, 1)
-                                   : apply_epi4<true>(x[i][j], p.epi, m, n);
-          __builtin_nontemporal_store(v, reinterpret_cast<f32x4 *>(p.Y + m * p.ldy + n));
-        }
-      }
-      return;
-    }
-  }
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -103,6 +67,116 @@ __global__ void elementwise_kernel(EltParams p) {
       const long m = m_base + i, n = n_base + j;
       if (m < p.M && n < p.N) p.Y[m * p.ldy + n] = apply_epi1(p.X[m * p.ldx + n], p.epi, m, (int)n);
     }
+}
+
+// Element ops on 16-byte aligned buffers, whatever the options' tiles: the
+// matrices are contiguous, so they are one stream of M * N elements, one 128-bit
+// vector per lane, and odd row lengths cost nothing (the bias column of a vector
+// is its element index mod N).  Bound by HBM.  Every byte is touched once, so
+// the accesses are non-temporal (cached ones: 1-8% slower on buffers that start
+// in HBM).  A workgroup's WAVES waves read as many segments of SEG KiB, 1 KiB each,
+// and consecutive workgroups walk the segments: workgroups that read 4 KiB in
+// one piece keep fewer HBM banks busy.  Back to back on cold buffers (us), one
+// piece / 8 waves x 32 KiB / 4 waves x 4 KiB: relu 2047x4093 12.4 / 11.3 / 11.7,
+// add 8192^2 124.0 / 119.1 / 119.2, relu 16384^2 324 / 313 / 307, add 16384^2
+// 499 / 481 / 469; so 8 x 32 below kHugeStream elements, 4 x 4 from there.
+// Against one element per thread on 16x16 tiles -> this: relu 2047x4093 27.8 ->
+// 11.3, add 4096^2 56.6 -> 31.5, add 8192^2 217 -> 119; against 1x4 elements on 4x256
+// tiles: relu 2047x4093 25.1 -> 11.3, relu 8192^2 80.2 -> 79.3, bias_add 8192^2
+// 81.6 -> 79.3 (6.77 TB/s).
+constexpr long kHugeStream = 1L << 27;
+constexpr long kMaxFlatGrid = 1L << 22;  // 2^32 elements in 4-wave workgroups
+
+// The bias of stream elements 4 * q .. + 3, the first in column n; columns wrap at
+// N (N may be 1).
+template <typename Idx>
+__device__ __forceinline__ f32x4 flat_bias(const float *bias, Idx n, Idx N) {
+  if (n + 4 <= N) return *reinterpret_cast<const f32x4_u *>(bias + n);
+  f32x4 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = bias[n];
+    n = n + 1 == N ? 0 : n + 1;
+  }
+  return v;
+}
+
+// Idx: unsigned where M * N < 2^32, else unsigned long.  ONE: the chain has at
+// most one bias and one add operand, which then arrive, like the op kinds (8
+// bits each in `kinds`), in preloaded arguments (13 SGPRs): a wave moves only
+// 2-4 KiB, and waiting for the epilogue's fields from the argument segment made
+// relu at 8192^2 78.7 -> 82.0 us, bias_add 80.0 -> 89.5.  `inv` = floor(2^32 / N).
+template <typename Idx, bool ONE, unsigned WAVES, unsigned SEG>
+__global__ void __launch_bounds__(64 * WAVES)
+elementwise_flat_kernel(const float *X, float *Y, long total, const float *bias, const float *R, unsigned N, unsigned inv,
+                        unsigned kinds, EltParams p) {
+  const unsigned lane = threadIdx.x & 63;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const Idx vecs = (Idx)((unsigned long)total / 4);
+  auto kind = [&](int i) __attribute__((always_inline)) { return (int)(kinds >> (8 * i)) & 255; };
+  auto body = [&](Idx b) __attribute__((always_inline)) {
+    const Idx piece = (b / SEG * WAVES + wave) * SEG + b % SEG;
+    const Idx q = piece * 64 + lane;
+    if (q >= vecs) return;
+    f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(X) + q);
+    // Column of this lane's first element: the wave's first column (scalar; the
+    // estimated quotient is the true one or one less), then at most one wrap
+    // where a row holds a wave's 256 elements.
+    auto column = [&]() __attribute__((always_inline)) {
+      const Idx e0 = piece * 256;
+      Idx n0;
+      if constexpr (sizeof(Idx) == 4) {
+        n0 = e0 - __umulhi(e0, inv) * N;
+        if (n0 >= N) n0 -= N;
+      } else {
+        n0 = e0 % N;
+      }
+      Idx n = n0 + 4 * lane;
+      if (N >= 256) return n >= N ? n - N : n;
+      return n % N;
+    };
+    // Every operand is requested before the first is used.
+    f32x4 r[ONE ? 2 : kMaxEpi];
+    if constexpr (ONE) {
+      if (bias) r[0] = flat_bias<Idx>(bias, column(), N);
+      if (R) r[1] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(R) + q);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kMaxEpi; ++i) {
+        if (kind(i) == EPI_BIAS) r[i] = flat_bias<Idx>(p.epi.ptr[i], column(), N);
+        else if (kind(i) == EPI_ADD) r[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(p.epi.ptr[i]) + q);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kMaxEpi; ++i) {
+      const int k = kind(i);
+      if (k == EPI_NONE) break;
+      if (k == EPI_BIAS) {
+        v += r[ONE ? 0 : i];
+      } else if (k == EPI_ADD) {
+        v += r[ONE ? 1 : i];
+      } else if (k == EPI_RELU) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = relu_ieee(v[e]);
+      } else if (k == EPI_ADD_SELF) {
+        v = v + v;
+      }
+    }
+    __builtin_nontemporal_store(v, reinterpret_cast<f32x4 *>(Y) + q);
+  };
+  if constexpr (sizeof(Idx) == 4) {
+    body(blockIdx.x);  // the grid covers every piece
+  } else {
+    constexpr Idx kSpan = 64 * WAVES * SEG;
+    for (Idx b = blockIdx.x; b < (vecs + kSpan - 1) / kSpan * SEG; b += gridDim.x) body(b);
+  }
+  // The last M * N mod 4 elements, one lane each.
+  if (blockIdx.x == 0 && threadIdx.x < (total & 3)) {
+    const long at = (total & ~3L) + threadIdx.x;
+    const long m = at / N;
+    const int n = (int)(at - m * N);
+    Y[at] = apply_epi1(X[at], p.epi, m, n);
+  }
 }
 
 template <int TM, int TN>
@@ -115,6 +189,34 @@ template <int TM, int TN>
 hipError_t launch_elementwise(const EltParams &p, dim3 grid, dim3 block, hipStream_t stream) {
   hipLaunchKernelGGL((elementwise_kernel<TM, TN>), grid, block, 0, stream, p);
   return hipGetLastError();
+}
+
+template <typename Idx, unsigned WAVES, unsigned SEG>
+static hipError_t launch_flat(const EltParams &p, const float *bias, const float *r, unsigned kinds, bool one,
+                              hipStream_t stream) {
+  const long total = (long)p.M * p.N, span = 64 * WAVES * SEG;
+  const long groups = std::max(1L, (total / 4 + span - 1) / span * SEG);
+  const unsigned n = (unsigned)p.N, inv = n > 1 ? (unsigned)((1UL << 32) / n) : ~0u;
+  auto fn = one ? &elementwise_flat_kernel<Idx, true, WAVES, SEG> : &elementwise_flat_kernel<Idx, false, WAVES, SEG>;
+  hipLaunchKernelGGL(fn, dim3((unsigned)std::min(groups, kMaxFlatGrid)), dim3(64 * WAVES), 0, stream, p.X, p.Y, total, bias,
+                     r, n, inv, kinds, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_elementwise_flat(const EltParams &p, hipStream_t stream) {
+  unsigned kinds = 0;
+  int biases = 0, adds = 0;
+  const float *bias = nullptr, *r = nullptr;
+  for (int i = 0; i < p.epi.nops; ++i) {
+    kinds |= (unsigned)p.epi.kind[i] << (8 * i);
+    if (p.epi.kind[i] == EPI_BIAS) bias = p.epi.ptr[i], ++biases;
+    if (p.epi.kind[i] == EPI_ADD) r = p.epi.ptr[i], ++adds;
+  }
+  const long total = (long)p.M * p.N;
+  const bool one = biases <= 1 && adds <= 1;
+  if (total < kHugeStream) return launch_flat<unsigned, 8, 32>(p, bias, r, kinds, one, stream);
+  if (total < (1L << 32)) return launch_flat<unsigned, 4, 4>(p, bias, r, kinds, one, stream);
+  return launch_flat<unsigned long, 4, 4>(p, bias, r, kinds, one, stream);
 }
 
 // Split-K reduction: one thread per 4 consecutive outputs; the partial-sum

@@ -383,13 +383,13 @@ int launch_stage(const tf_kernel *k, size_t s, void *const *ptrs, void *ws, hipS
     p.ldx = st.N;
     p.ldy = st.N;
     p.epi = make_epi(st, ptrs);
-    bool vec = st.N % 4 == 0;
+    // The flat kernel on aligned buffers (the bias, read by column, needs no
+    // alignment); the options' own geometry on the rest.
     auto aligned = [](const void *q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
-    vec = vec && aligned(p.X) && aligned(p.Y);
+    bool flat = aligned(p.X) && aligned(p.Y);
     for (int i = 0; i < p.epi.nops; ++i)
-      if (p.epi.ptr[i]) vec = vec && aligned(p.epi.ptr[i]);
-    p.vec_ok = vec ? 1 : 0;
-    err = L.entry->elt(p, L.grid, L.block, stream);
+      if (p.epi.kind[i] == tfk::EPI_ADD) flat = flat && aligned(p.epi.ptr[i]);
+    err = flat ? tfk::launch_elementwise_flat(p, stream) : L.entry->elt(p, L.grid, L.block, stream);
   }
   if (err != hipSuccess)
     return fail(TF_E_HIP, std::string("kernel launch ") + L.entry->name + " failed: " + hipGetErrorString(err));

@@ -62,7 +62,6 @@ struct EltParams {
   int M, N;
   long ldx, ldy;
   EpiParams epi;
-  int vec_ok;  // 1: every operand 16-byte aligned with row strides a multiple of 4
 };
 
 enum Family : int { FAM_DIRECT = 0, FAM_STAGED = 1, FAM_ELEMENTWISE = 2, FAM_WAVEK = 4 };
@@ -82,6 +81,10 @@ struct KernelEntry {
   EltLauncher elt;
   int lds_bytes;   // static LDS of the instantiation
 };
+
+// Element ops over contiguous operands (row strides N): X, Y and the add operands
+// 16-byte aligned, biases at any alignment (direct_kernels.hip).
+hipError_t launch_elementwise_flat(const EltParams &p, hipStream_t stream);
 
 // The split-K reduction (direct_kernels.hip); ws and C 16-byte aligned.
 hipError_t launch_splitk_reduce(const ReduceParams &p, hipStream_t stream);
