@@ -39,11 +39,7 @@
 //    middle of slab t+2), so the LDS writes do not wait on HBM latency under
 //    full-chip load (one set, 1.5 slabs ahead, for the register-heavy
 //    configurations); the slab loop is unrolled by two so buffer and set
-//    indices are compile-time.  (The loads are conditional near the end of
-//    K, so the compiler's wait before every other slab's stores covers both
-//    sets; loads issued a slab earlier have landed by then, and clamped
-//    unconditional loads with exact waits measured no faster.)  The barrier sits before the slab's last
-//    chunk so those MFMAs hide the next slab's first LDS reads.  Each
+//    indices are compile-time.  The barrier sits before the slab's last chunk so those MFMAs hide the next slab's first LDS reads.  Each
 //    chunk's MFMAs are scheduled around the next chunk's fragment reads in a
 //    measured order.  Row padding makes the b128 fragment reads and the b32
 //    B reads bank-conflict-free.
@@ -89,7 +85,10 @@ __device__ __forceinline__ AccOf<MB> mfma_block(float b, float a, AccOf<MB> c) {
 // Output tile (tm, tn) of linear tile index w on a gx x gy tile grid.  With
 // swizzle, consecutive w are dealt to the 8 XCDs round-robin (as the hardware
 // deals workgroups), so the indices one XCD receives are remapped to a
-// compact block of tiles, grouped by 4 tile rows.
+// compact block of tiles, grouped by 4 tile rows.  For every tile count: left in
+// row-major order where 8 does not divide it, masked 64x64 t4x4 k16 tiles ran
+// 98.0 us instead of 86.7 at 2100x3300x700 and 119 instead of 96.5 at 1700x3500x900.
+// Groups of 8 rows were no faster (4095x4097x1023 301 against 294).
 __device__ __forceinline__ void tile_coords(int w, int gx, int gy, int swizzle, int &tm, int &tn) {
   const int total = gx * gy;
   if (!swizzle) {
@@ -98,7 +97,9 @@ __device__ __forceinline__ void tile_coords(int w, int gx, int gy, int swizzle, 
     return;
   }
   constexpr int kXcds = 8;
-  if (total % kXcds == 0) w = (w % kXcds) * (total / kXcds) + w / kXcds;
+  // (The first total % 8 XCDs get one tile more.)
+  const int x = w % kXcds;
+  w = x * (total / kXcds) + min(x, total % kXcds) + w / kXcds;
   constexpr int kGroup = 4;
   const int group = w / (kGroup * gx);
   const int first = group * kGroup;
@@ -124,9 +125,10 @@ __device__ __forceinline__ void static_for(F &&f) {
 // One staging vector (a float or a 4-vector) by a raw buffer load at a byte
 // offset from the resource's base.
 template <typename VT>
-__device__ __forceinline__ VT buffer_load_vt(__amdgpu_buffer_rsrc_t rs, int byte_off) {
-  if constexpr (sizeof(VT) == 16) return __builtin_bit_cast(VT, __builtin_amdgcn_raw_buffer_load_b128(rs, byte_off, 0, 0));
-  else return __builtin_bit_cast(VT, __builtin_amdgcn_raw_buffer_load_b32(rs, byte_off, 0, 0));
+__device__ __forceinline__ VT buffer_load_vt(__amdgpu_buffer_rsrc_t rs, int byte_off, int scalar_off = 0) {
+  if constexpr (sizeof(VT) == 16)
+    return __builtin_bit_cast(VT, __builtin_amdgcn_raw_buffer_load_b128(rs, byte_off, scalar_off, 0));
+  else return __builtin_bit_cast(VT, __builtin_amdgcn_raw_buffer_load_b32(rs, byte_off, scalar_off, 0));
 }
 
 // Write element e of a staging register (a float or a 4-vector).
@@ -332,18 +334,13 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     // `gm` (std::integral_constant<int, 0 or 1>): 0 when the caller knows
     // the slab is not guarded (the masked kernels' steady state, see the slab
     // loop), so the guarded branch is not compiled in.
-    // Buffer loads (`bc` = BufOn; unmasked staging, and the masked kernels'
-    // unguarded slabs): the slab's base addresses go into two buffer
-    // resources (scalar 64-bit arithmetic) and each thread keeps one 32-bit
-    // byte offset per vector, so a global load carries no 64-bit vector
-    // address add.  Between the MFMAs of one wave per
-    // SIMD those adds cost 1.5 us at 1024^3 (64x64 t4x4 k16: 19.3 -> 17.75 us
-    // back to back) and 6 us at 2048^3 (128x128 t8x8 k16: 126.4 -> 120.0 us).
-    // Used only when every offset fits 31 bits (the caller checks BM * lda and
-    // BK * ldb); otherwise the same loop runs with flat loads.  Masked
-    // kernels: A rows clamped to M - 1 as in their flat loads, offsets from
-    // the tile's first row; B columns are absolute (clamped to N - 4), so B's
-    // base is the slab's first row of the matrix.
+    // Buffer loads (`bc` = BufOn; unmasked block-staged kernels): the slab's
+    // base addresses go into two buffer resources (scalar 64-bit arithmetic) and
+    // each thread keeps one 32-bit byte offset per vector, so a global load
+    // carries no 64-bit vector address add (128x128 t8x4 k32 at 2048^3 124.9 ->
+    // 123.6 us).  Used only when every offset fits 31 bits (the caller checks
+    // BM * lda and BK * ldb); otherwise the same loop runs with flat loads.  (The
+    // kernels that spread their staging use bounded loads, below.)
     using BufOn = std::integral_constant<int, 1>;
     using BufOff = std::integral_constant<int, 0>;
     auto buf_rsrc = [](const float *base) __attribute__((always_inline)) {
@@ -352,20 +349,15 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     auto a_byte = [&](int it) __attribute__((always_inline)) {
       int r, c;
       G::a_item(tid + it * NT, r, c);
-      if constexpr (MASK) r = min(m0i + r, Mi - 1) - m0i;
       return (int)((r * lda + c) * 4);
     };
     auto b_byte = [&](int it) __attribute__((always_inline)) {
-      if constexpr (MASK) return (b_off[it] - kbi * (int)ldb) * 4;
       const int q = tid + it * NT, r = q / (BN / VW), c = (q - r * (BN / VW)) * VW;
       return (int)((r * ldb + c) * 4);
     };
-    auto b_base = [&](int k0) __attribute__((always_inline)) {
-      return MASK ? p.B + (kbase + k0) * ldb : B + (long)k0 * ldb;
-    };
     auto buf_slab = [&](auto sc, int k0) __attribute__((always_inline)) {
       constexpr int set = decltype(sc)::value;
-      const __amdgpu_buffer_rsrc_t rsa = buf_rsrc(A + k0), rsb = buf_rsrc(b_base(k0));
+      const __amdgpu_buffer_rsrc_t rsa = buf_rsrc(A + k0), rsb = buf_rsrc(B + (long)k0 * ldb);
 #pragma unroll
       for (int it = 0; it < G::A_PER; ++it)
         if (G::A_VECS % NT == 0 || tid + it * NT < G::A_VECS) ra[set][it] = buffer_load_vt<VT>(rsa, a_byte(it));
@@ -393,10 +385,6 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
           if (G::B_VECS % NT == 0 || q < G::B_VECS) rb[set][it] = *reinterpret_cast<const VT *>(b_src[it] + k0 * ldb);
         }
       } else if (decltype(gm)::value == 0 || !guarded(k0)) {
-        if constexpr (decltype(bc)::value) {
-          buf_slab(sc, k0);
-          return;
-        }
 #pragma unroll
         for (int it = 0; it < G::A_PER; ++it) {
           const int q = tid + it * NT;
@@ -483,6 +471,61 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
       }
     };
 
+    // Bounded loads (kernels that spread their staging): the buffer resources
+    // end where the matrices do, and a buffer load returns zero for each of its
+    // dwords past the end without touching memory.  Rows of A past M, rows of B
+    // past K and whole slabs past this workgroup's K range load as zeros with the
+    // same instructions as every other slab; only A's columns past K (its next
+    // row) have to be cleared, in the registers, on the way to LDS (the last
+    // slabs, `gm` = 3).  So every slab runs the same straight-line code, with exact
+    // waits and no tail of conditional loads.  The resources stay as they are
+    // through the loop: the slab's offset is the load's scalar offset, which the
+    // bounds check includes, so a slab costs two scalar additions.  (Resources
+    // rebuilt from k0 every slab took 45 scalar instructions, which with one wave
+    // per SIMD do not fit beside an MFMA: masked 1000^3 25.0 us.)  Against
+    // flat or per-slab buffer loads with guarded, conditional tails, us back to
+    // back: masked 64x64 t4x4 k16 777x1111x333 10.9 -> 9.9, 1000^3 20.0 -> 18.8,
+    // 4095x4097x1023 274 -> 270; unmasked 32x32 t2x2 k32 512^3 5.34 -> 4.98,
+    // 512x512x2048 12.0 -> 11.2, 64x64 t4x4 k16 1024^3 18.2 -> 17.95; 128x128 t8x8
+    // k16 2048^3 120.5 -> 120.4.  VGPRs of the masked kernels: 99 -> 66 (64x64),
+    // 171 -> 113 (128x128).
+    __amdgpu_buffer_rsrc_t rsa, rsb;
+    int off_a = 0, off_b = 0;  // byte offsets of the next slab to load
+    const int b_step = BK * (int)ldb * 4;
+    constexpr long kBufElems = 1L << 29;  // 31-bit byte offsets
+    // B's resource from row `row` of this workgroup's K range on.
+    auto bound_b = [&](int row) __attribute__((always_inline)) {
+      const long elems = (min(Ki - kbi, nk * BK) - row) * ldb - n0;
+      rsb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(B + row * ldb), 0,
+                                              (int)max(0L, min(elems, kBufElems - 1)) * 4, 0x00020000);
+      off_b = 0;
+    };
+    auto load_bounded = [&](auto sc, auto qc) __attribute__((always_inline)) {
+      constexpr int set = decltype(sc)::value, it = decltype(qc)::value;
+      if constexpr (it < G::A_PER) {
+        int r, c;
+        G::a_item(tid + it * NT, r, c);
+        if (G::A_VECS % NT == 0 || tid + it * NT < G::A_VECS)
+          ra[set][it] = buffer_load_vt<VT>(rsa, (int)((r * lda + c) * 4), off_a);
+      } else {
+        constexpr int ib = it - G::A_PER;
+        const int q = tid + ib * NT, r = q / (BN / VW), c = (q - r * (BN / VW)) * VW;
+        if (G::B_VECS % NT == 0 || q < G::B_VECS) rb[set][ib] = buffer_load_vt<VT>(rsb, (int)((r * ldb + c) * 4), off_b);
+      }
+    };
+    // Clears the columns of A at or past K in staging vector `it` of slab k0.
+    auto clear_k_tail = [&](auto sc, auto qc, int k0) __attribute__((always_inline)) {
+      constexpr int set = decltype(sc)::value, it = decltype(qc)::value;
+      if constexpr (it < G::A_PER) {
+        int r, c;
+        G::a_item(tid + it * NT, r, c);
+        const int left = Ki - kbi - k0 - c;
+#pragma unroll
+        for (int e = 0; e < VW; ++e)
+          if (e >= left) put(ra[set][it], e, SEQ ? -0.0f : 0.0f);
+      }
+    };
+
     // Schedule per slab t (slab t lives in buffer t & 1, C = BK / KC chunks):
     //   chunk kc:     read chunk kc+1's fragments, then chunk kc's MFMAs
     //   chunk C/2-1:  after its MFMAs, store slab t+1 (registers, loaded one
@@ -516,18 +559,9 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     float bf[2][FN][4];
     // One staging vector (item q < A_PER: A, else B) of a slab that is not
     // guarded (the loads of load_slab's unmasked and unguarded paths).
-    auto load_item = [&](auto sc, auto qc, int k0, auto bc) __attribute__((always_inline)) {
+    auto load_item = [&](auto sc, auto qc, int k0) __attribute__((always_inline)) {
       constexpr int set = decltype(sc)::value, it = decltype(qc)::value;
-      if constexpr (decltype(bc)::value) {
-        if constexpr (it < G::A_PER) {
-          if (G::A_VECS % NT == 0 || tid + it * NT < G::A_VECS)
-            ra[set][it] = buffer_load_vt<VT>(buf_rsrc(A + k0), a_byte(it));
-        } else {
-          constexpr int ib = it - G::A_PER;
-          if (G::B_VECS % NT == 0 || tid + ib * NT < G::B_VECS)
-            rb[set][ib] = buffer_load_vt<VT>(buf_rsrc(b_base(k0)), b_byte(ib));
-        }
-      } else if constexpr (it < G::A_PER) {
+      if constexpr (it < G::A_PER) {
         const int q = tid + it * NT;
         if (G::A_VECS % NT == 0 || q < G::A_VECS) {
           int r, c;
@@ -581,29 +615,35 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
 #pragma unroll
         for (int s = 0; s < 4; ++s) bf[slot][j][s] = bs[s * G::B_ROW_S * LDB + j * MB];
     };
-    // Slab 0's loads go out first: the bias test reads the epilogue fields
-    // from the kernel-argument segment, and its wait would delay them.
-    if (nk > 0) load_slab(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, 0, BufOff{});
-    if (bias_early && tid < BN / 4)
-      *reinterpret_cast<f32x4 *>(&bias_s[4 * tid]) = *reinterpret_cast<const f32x4 *>(p.epi.ptr[0] + n0 + 4 * tid);
-    if (nk > 0) {
-      store_slab(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, 0, 0);
-      if (nk > 1) load_slab(std::integral_constant<int, DEPTH - 1>{}, std::integral_constant<int, 1>{}, BK, BufOff{});
-      if (DEPTH == 2 && nk > 2)
-        load_slab(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, 2 * BK, BufOff{});
-    }
-    __syncthreads();
-    if (nk > 0) load_frags(0, 0, 0);
+    auto stage_bias = [&]() __attribute__((always_inline)) {
+      if (bias_early && tid < BN / 4)
+        *reinterpret_cast<f32x4 *>(&bias_s[4 * tid]) = *reinterpret_cast<const f32x4 *>(p.epi.ptr[0] + n0 + 4 * tid);
+    };
+    auto prologue = [&]() __attribute__((always_inline)) {
+      // Slab 0's loads go out first: the bias test reads the epilogue fields
+      // from the kernel-argument segment, and its wait would delay them.
+      if (nk > 0) load_slab(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, 0, BufOff{});
+      stage_bias();
+      if (nk > 0) {
+        store_slab(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, 0, 0);
+        if (nk > 1) load_slab(std::integral_constant<int, DEPTH - 1>{}, std::integral_constant<int, 1>{}, BK, BufOff{});
+        if (DEPTH == 2 && nk > 2)
+          load_slab(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, 2 * BK, BufOff{});
+      }
+      __syncthreads();
+      if (nk > 0) load_frags(0, 0, 0);
+    };
     // One slab; P = kt & 1 names its LDS buffer; slab s is staged in set
     // s & 1 (two sets) or 0 (one set), and slab kt + 1 + DEPTH is loaded into
     // the set that slab kt + 1 leaves.
     // `gm` = 0: a masked kernel's steady state, where every slab this one
     // stores or loads is unguarded and a next slab exists (see the loop
     // below), so the loads are unconditional and the compiler's waits exact.
+    // `gm` = 2: bounded loads; 3: and A's K tail cleared in the slab it stores.
     auto slab = [&](auto par, auto gm, int kt, auto bc) __attribute__((always_inline)) {
       constexpr int P = decltype(par)::value;
       constexpr int cur = P;
-      constexpr bool steady = decltype(gm)::value == 0;
+      constexpr bool steady = decltype(gm)::value != 1, bounded = decltype(gm)::value >= 2;
       const bool more = steady || kt + 1 < nk;
 #pragma unroll
       for (int kc = 0; kc < C; ++kc) {
@@ -632,11 +672,16 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
               static_for<2 * NSTG>([&](auto oc) __attribute__((always_inline)) {
                 constexpr int o = decltype(oc)::value;
                 if (o == op) {
-                  if constexpr (o % 2 == 0)
+                  if constexpr (o % 2 == 0) {
+                    if constexpr (decltype(gm)::value == 3)
+                      clear_k_tail(std::integral_constant<int, SET>{}, std::integral_constant<int, o / 2>{}, (kt + 1) * BK);
                     store_item(std::integral_constant<int, SET>{}, std::integral_constant<int, o / 2>{}, cur ^ 1);
-                  else
+                  } else if constexpr (bounded) {
+                    load_bounded(std::integral_constant<int, SET>{}, std::integral_constant<int, o / 2>{});
+                  } else {
                     load_item(std::integral_constant<int, SET>{}, std::integral_constant<int, o / 2>{},
-                              (kt + 1 + DEPTH) * BK, bc);
+                              (kt + 1 + DEPTH) * BK);
+                  }
                 }
               });
               __builtin_amdgcn_sched_barrier(0);
@@ -690,6 +735,10 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
             load_slab(std::integral_constant<int, DEPTH == 2 ? (P ^ 1) : 0>{}, gm, (kt + 1 + DEPTH) * BK, bc);
         }
       }
+      if constexpr (bounded) {
+        off_a += BK * 4;
+        off_b += b_step;
+      }
       // With an odd chunk count the next slab's first fragments landed in
       // slot 1; the loop expects them in slot 0.
       if constexpr (C % 2 == 1) {
@@ -728,18 +777,71 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
       }
       if (kt < nk) slab(std::integral_constant<int, 0>{}, Any{}, kt, bc);
     };
-    // Buffer loads where measured faster: the spread kernels, and the
-    // block-staged ones with tiles of at least 128 x 128 (2048^3 t8x4 k32
-    // 124.9 -> 123.6 us; the 8-wave 64x64 t4x2 k64 at 1024^3 was 2.4% slower
-    // with them).  Not for 1024-thread workgroups (128 VGPRs per lane): the
-    // flat-load copy of the loop beside the buffer one spills there; masked
-    // kernels only where they spread their staging (the block-staged masked
-    // ones with 512 threads and tile-k 32 or 64 spill with both loops).
-    constexpr bool BUFCAP = VEC && NT < 1024 && (SPREAD || (!MASK && BM * BN >= 128 * 128));
-    if constexpr (BUFCAP) {
-      if ((long)BM * lda + BK < (1L << 29) && (long)BK * ldb + (MASK ? Ni : BN) < (1L << 29)) k_loop(BufOn{});
+    // Bounded loads for the spread kernels; per-slab buffer loads for unmasked
+    // block-staged tiles of at least 128 x 128 (2048^3 t8x4 k32 124.9 -> 123.6 us;
+    // the 8-wave 64x64 t4x2 k64 at 1024^3 was 2.4% slower with them).  Not for
+    // 1024-thread workgroups (128 VGPRs per lane): the flat-load copy of the loop
+    // beside the buffer one spills there, as it does in masked block-staged
+    // kernels with 512 threads and tile-k 32 or 64.
+    if constexpr (SPREAD) {
+      // (Six slabs of B at least: three in flight, two computed per iteration.)
+      if ((long)BM * lda + BK < kBufElems && 6L * BK * ldb + BN < kBufElems) {
+        // Slab t is staged in register set t & 1.
+        using Bounded = std::integral_constant<int, 2>;
+        using Last = std::integral_constant<int, MASK ? 3 : 2>;
+        using Set0 = std::integral_constant<int, 0>;
+        using Set1 = std::integral_constant<int, 1>;
+        const int a_elems = (MASK ? min(Mi - m0i, BM) : BM) * (int)lda - kbi;
+        rsa = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, a_elems * 4, 0x00020000);
+        bound_b(0);
+        auto load_all = [&](auto sc) __attribute__((always_inline)) {
+          static_for<NSTG>([&](auto qc) __attribute__((always_inline)) { load_bounded(sc, qc); });
+          off_a += BK * 4;
+          off_b += b_step;
+        };
+        load_all(Set0{});
+        load_all(Set1{});
+        stage_bias();
+        static_for<NSTG>([&](auto qc) __attribute__((always_inline)) {
+          if constexpr (MASK) clear_k_tail(Set0{}, qc, 0);
+          store_item(Set0{}, qc, 0);
+        });
+        load_all(Set0{});
+        __syncthreads();
+        load_frags(0, 0, 0);
+        // B is walked in windows that 31-bit offsets reach: one unless this
+        // workgroup's K range of it exceeds 2 GiB.  From slab `end` on there is
+        // nothing left to load (A's resource is emptied: the next slabs would be
+        // real memory, the start of its next rows) and masked kernels store the K
+        // tail.
+        const int end = nk - 3;
+        const int window = (Ki + 4L * BK) * ldb + BN < kBufElems ? nk : (int)((kBufElems - BN) / ((long)BK * ldb) - 4) & ~1;
+        int kt = 0;
+        for (;;) {
+          const int stop = min(end, kt + window);
+          for (; kt < stop; kt += 2) {
+            slab(Set0{}, Bounded{}, kt, BufOn{});
+            slab(Set1{}, Bounded{}, kt + 1, BufOn{});
+          }
+          if (kt >= end) break;
+          bound_b((kt + 3) * BK);
+        }
+        rsa = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, 0, 0x00020000);
+        for (; kt + 1 < nk; kt += 2) {
+          slab(Set0{}, Last{}, kt, BufOn{});
+          slab(Set1{}, Last{}, kt + 1, BufOn{});
+        }
+        if (kt < nk) slab(Set0{}, Bounded{}, kt, BufOn{});
+      } else {
+        prologue();
+        k_loop(BufOff{});
+      }
+    } else if constexpr (VEC && NT < 1024 && !MASK && BM * BN >= 128 * 128) {
+      prologue();
+      if ((long)BM * lda + BK < kBufElems && (long)BK * ldb + BN < kBufElems) k_loop(BufOn{});
       else k_loop(BufOff{});
     } else {
+      prologue();
       k_loop(BufOff{});
     }
   } else {
