@@ -218,7 +218,7 @@ def main(shards=16):
             lines.append(f"    KernelEntry{{FAM_STAGED, {t}, \"{name(c)}\",")
             lines.append(f"                reinterpret_cast<const void *>(&staged_gemm_kernel<{t}>),")
             t7 = ", ".join(str(x) for x in c[:7])
-            lines.append(f"                &launch_staged<{t}>, nullptr, StagedGemm<{t7}>::LDS_BYTES}},")
+            lines.append(f"                &launch_staged<{t}>, nullptr, StagedGemm<{t7}, 0, {c[7]}>::LDS_BYTES}},")
         lines += ["};", f"extern const int kStagedCount{i} = {len(part)};", "#else",
                   "// Device pass: instantiate the kernels the host table names."]
         for c in part:

@@ -135,7 +135,7 @@ __device__ __forceinline__ VT buffer_load_vt(__amdgpu_buffer_rsrc_t rs, int byte
 __device__ __forceinline__ void put(float &v, int, float x) { v = x; }
 __device__ __forceinline__ void put(f32x4 &v, int e, float x) { v[e] = x; }
 
-template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC, int SEQ = 0>
+template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC, int SEQ = 0, int MASK = 0>
 struct StagedGemm {
   static constexpr int NT = (BM / TM) * (BN / TN);
   static constexpr int WTM = 8 * TM, WTN = 8 * TN;
@@ -158,7 +158,12 @@ struct StagedGemm {
   static constexpr int B_ROW_G = SEQ ? 1 : 4, B_ROW_S = SEQ ? 64 / MB : 1;
   static constexpr int A_ELEMS = BM * LDA, B_ELEMS = BK * LDB;
   // Two A and B tile buffers, plus the tile's BN bias values.
-  static constexpr int LDS_BYTES = PROMOTE ? 2 * (A_ELEMS + B_ELEMS) * 4 + BN * 4 : 0;
+  // Masked 64x64 t4x4 k16 (CROWD): padded to four workgroups per CU.  A slab is
+  // half of each 128-byte line of its A rows; six workgroups' lines outlive
+  // the L1 before the next slab wants the other half.
+  static constexpr bool CROWD = MASK && !SEQ && PROMOTE && VEC && BM == 64 && BN == 64 && TM == 4 && TN == 4 && BK == 16;
+  static constexpr int CROWD_PAD = CROWD ? 13312 / 4 : 0;
+  static constexpr int LDS_BYTES = PROMOTE ? 2 * (A_ELEMS + B_ELEMS) * 4 + (BN + CROWD_PAD) * 4 : 0;
   // Global -> register staging per thread and slab.
   static constexpr int VW = VEC ? 4 : 1;
   static constexpr int A_VECS = BM * BK / VW, B_VECS = BK * BN / VW;
@@ -232,7 +237,7 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
   p.N = pN;
   p.swizzle = flags & 255;
   p.splits = flags >> 8;
-  using G = StagedGemm<BM, BN, TM, TN, BK, PROMOTE, VEC, SEQ>;
+  using G = StagedGemm<BM, BN, TM, TN, BK, PROMOTE, VEC, SEQ, MASK>;
   constexpr int NT = G::NT, WTM = G::WTM, WTN = G::WTN, NWN = G::NWN, FM = G::FM, FN = G::FN;
   constexpr int LDA = G::LDA, LDB = G::LDB, VW = G::VW, MB = G::MB, KC = G::KC;
   using AccT = AccOf<MB>;
@@ -278,7 +283,7 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
   // epilogue reads them from LDS instead of starting on a cold global load.
   // Not for split-K (the reduction applies the epilogue) or edge tiles
   // (their columns may leave the matrix).
-  __shared__ __attribute__((aligned(16))) float bias_s[BN];
+  __shared__ __attribute__((aligned(16))) float bias_s[BN + G::CROWD_PAD];
   const bool bias_early = PROMOTE && splits == 1 && !edge && p.epi.nops > 0 && p.epi.kind[0] == EPI_BIAS;
 
   if constexpr (PROMOTE) {
@@ -639,7 +644,8 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     // `gm` = 0: a masked kernel's steady state, where every slab this one
     // stores or loads is unguarded and a next slab exists (see the loop
     // below), so the loads are unconditional and the compiler's waits exact.
-    // `gm` = 2: bounded loads; 3: and A's K tail cleared in the slab it stores.
+    // `gm` = 2: bounded loads; 3: and A's K tail cleared in the slab it stores;
+    // 4: and all but the newest load waited for before the first store.
     auto slab = [&](auto par, auto gm, int kt, auto bc) __attribute__((always_inline)) {
       constexpr int P = decltype(par)::value;
       constexpr int cur = P;
@@ -673,6 +679,7 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
                 constexpr int o = decltype(oc)::value;
                 if (o == op) {
                   if constexpr (o % 2 == 0) {
+                    if constexpr (o == 0 && decltype(gm)::value == 4) __builtin_amdgcn_s_waitcnt(0x0f71);  // vmcnt(1)
                     if constexpr (decltype(gm)::value == 3)
                       clear_k_tail(std::integral_constant<int, SET>{}, std::integral_constant<int, o / 2>{}, (kt + 1) * BK);
                     store_item(std::integral_constant<int, SET>{}, std::integral_constant<int, o / 2>{}, cur ^ 1);
@@ -817,12 +824,23 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
         const int end = nk - 3;
         const int window = (Ki + 4L * BK) * ldb + BN < kBufElems ? nk : (int)((kBufElems - BN) / ((long)BK * ldb) - 4) & ~1;
         int kt = 0;
+        auto steady = [&](auto mode, int stop) __attribute__((always_inline)) {
+          for (; kt < stop; kt += 2) {
+            slab(Set0{}, mode, kt, BufOn{});
+            slab(Set1{}, mode, kt + 1, BufOn{});
+          }
+        };
+        // More workgroups than the four a CU holds: their loads crowd the memory
+        // path, and waiting a slab earlier (the other workgroups compute
+        // meanwhile) is faster: 4095x4097x1023 283 -> 277 us, against 280 with
+        // guarded loads.  With fewer it only waits: 777x1111x333 10.0 -> 10.8.
+        const bool crowded = G::CROWD && gx * gy > 4 * 256;
         for (;;) {
           const int stop = min(end, kt + window);
-          for (; kt < stop; kt += 2) {
-            slab(Set0{}, Bounded{}, kt, BufOn{});
-            slab(Set1{}, Bounded{}, kt + 1, BufOn{});
+          if constexpr (G::CROWD) {
+            if (crowded) steady(std::integral_constant<int, 4>{}, stop);
           }
+          if (!crowded) steady(Bounded{}, stop);
           if (kt >= end) break;
           bound_b((kt + 3) * BK);
         }
