@@ -131,6 +131,65 @@ __device__ __forceinline__ VT buffer_load_vt(__amdgpu_buffer_rsrc_t rs, int byte
   else return __builtin_bit_cast(VT, __builtin_amdgcn_raw_buffer_load_b32(rs, byte_off, scalar_off, 0));
 }
 
+// Where a bounded-load kernel's next slab of A and B is: byte offsets into their
+// buffer resources, used as the loads' scalar offsets (host code too, so that a
+// test can walk them).  The range check subtracts the scalar offset from the
+// resource's size, so it has to stay below the size: only a load's vector offset
+// may leave the matrix.  The prologue loads three slabs whatever nk is, and the loop,
+// two slabs per iteration and three ahead, may ask for slab nk; both ask for the
+// last slab again instead (in a cache by now; the values are never used).
+struct SlabOffsets {
+  int a = 0, b = 0, last_a = 0, last_b = 0;
+  // B's resource starts at slab `first` of this workgroup's `nk`.
+  __host__ __device__ __forceinline__ void rebase(int first, int nk, int a_step, int b_step) {
+    const long rest = (long)(nk - 1 - first) * b_step;
+    b = 0;
+    last_a = nk > 1 ? (nk - 1) * a_step : 0;
+    last_b = rest < 0 ? 0 : rest < 0x7fffffffL ? (int)rest : 0x7fffffff;
+  }
+  // After the prologue's loads and after a slab whose index is P mod 2.  (Slab nk
+  // follows an even slab: the pairs start at even slabs and stop past slab nk - 1.)
+  template <int P>
+  __host__ __device__ __forceinline__ void next(int a_step, int b_step) {
+    a += a_step;
+    b += b_step;
+    if constexpr (P == 0) {
+      a = a < last_a ? a : last_a;
+      b = b < last_b ? b : last_b;
+    }
+  }
+};
+
+// Walks nk slabs, kt being the next to compute (0 on entry): three loads ahead,
+// then pairs of slabs that load, in windows of `window` slabs of B, then at most
+// three slabs that load nothing.
+//   load(set)    slabs 0, 1 and 2 into register sets 0, 1 and 0
+//   first()      slab 0 to LDS
+//   ready()      the barrier, and slab 0's first fragments
+//   steady(stop) slabs kt and kt + 1, each loading the slab three on, until kt >= stop
+//   rebase(t)    B's resource from slab t on
+//   pair(), last()  slabs kt and kt + 1; slab kt = nk - 1
+template <typename Load, typename First, typename Ready, typename Steady, typename Rebase, typename Pair, typename Last>
+__host__ __device__ __forceinline__ void walk_slabs(int nk, int window, int &kt, Load &&load, First &&first, Ready &&ready,
+                                                    Steady &&steady, Rebase &&rebase, Pair &&pair, Last &&last) {
+  load(std::integral_constant<int, 0>{});
+  load(std::integral_constant<int, 1>{});
+  first();
+  load(std::integral_constant<int, 0>{});
+  ready();
+  const int end = nk - 3;  // slab end - 1 loads slab nk - 1
+  for (;;) {
+    steady(end < kt + window ? end : kt + window);
+    if (kt >= end) break;
+    rebase(kt + 3);
+  }
+  if (kt + 1 < nk) {
+    pair();
+    kt += 2;
+  }
+  if (kt < nk) last();
+}
+
 // Write element e of a staging register (a float or a 4-vector).
 __device__ __forceinline__ void put(float &v, int, float x) { v = x; }
 __device__ __forceinline__ void put(f32x4 &v, int e, float x) { v[e] = x; }
@@ -479,12 +538,12 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     // Bounded loads (kernels that spread their staging): the buffer resources
     // end where the matrices do, and a buffer load returns zero for each of its
     // dwords past the end without touching memory.  Rows of A past M, rows of B
-    // past K and whole slabs past this workgroup's K range load as zeros with the
+    // past K load as zeros with the
     // same instructions as every other slab; only A's columns past K (its next
-    // row) have to be cleared, in the registers, on the way to LDS (the last
-    // slabs, `gm` = 3).  So every slab runs the same straight-line code, with exact
-    // waits and no tail of conditional loads.  The resources stay as they are
-    // through the loop: the slab's offset is the load's scalar offset, which the
+    // row) have to be cleared, in the registers, on the way to LDS (the closing
+    // slabs, `gm` = 3).  So every slab that loads runs the same straight-line code,
+    // with exact waits and no tail of conditional loads.  The resources stay as they
+    // are through the loop: the slab's offset is the load's scalar offset, which the
     // bounds check includes, so a slab costs two scalar additions.  (Resources
     // rebuilt from k0 every slab took 45 scalar instructions, which with one wave
     // per SIMD do not fit beside an MFMA: masked 1000^3 25.0 us.)  Against
@@ -495,15 +554,16 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     // k16 2048^3 120.5 -> 120.4.  VGPRs of the masked kernels: 99 -> 66 (64x64),
     // 171 -> 113 (128x128).
     __amdgpu_buffer_rsrc_t rsa, rsb;
-    int off_a = 0, off_b = 0;  // byte offsets of the next slab to load
-    const int b_step = BK * (int)ldb * 4;
+    SlabOffsets at;  // scalar offsets of the next slab to load
+    const int a_step = BK * 4, b_step = BK * (int)ldb * 4;
     constexpr long kBufElems = 1L << 29;  // 31-bit byte offsets
-    // B's resource from row `row` of this workgroup's K range on.
-    auto bound_b = [&](int row) __attribute__((always_inline)) {
+    // B's resource from slab `first` of this workgroup's K range on.
+    auto bound_b = [&](int first) __attribute__((always_inline)) {
+      const int row = first * BK;
       const long elems = (min(Ki - kbi, nk * BK) - row) * ldb - n0;
       rsb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(B + row * ldb), 0,
                                               (int)max(0L, min(elems, kBufElems - 1)) * 4, 0x00020000);
-      off_b = 0;
+      at.rebase(first, nk, a_step, b_step);
     };
     auto load_bounded = [&](auto sc, auto qc) __attribute__((always_inline)) {
       constexpr int set = decltype(sc)::value, it = decltype(qc)::value;
@@ -511,11 +571,11 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
         int r, c;
         G::a_item(tid + it * NT, r, c);
         if (G::A_VECS % NT == 0 || tid + it * NT < G::A_VECS)
-          ra[set][it] = buffer_load_vt<VT>(rsa, (int)((r * lda + c) * 4), off_a);
+          ra[set][it] = buffer_load_vt<VT>(rsa, (int)((r * lda + c) * 4), at.a);
       } else {
         constexpr int ib = it - G::A_PER;
         const int q = tid + ib * NT, r = q / (BN / VW), c = (q - r * (BN / VW)) * VW;
-        if (G::B_VECS % NT == 0 || q < G::B_VECS) rb[set][ib] = buffer_load_vt<VT>(rsb, (int)((r * ldb + c) * 4), off_b);
+        if (G::B_VECS % NT == 0 || q < G::B_VECS) rb[set][ib] = buffer_load_vt<VT>(rsb, (int)((r * ldb + c) * 4), at.b);
       }
     };
     // Clears the columns of A at or past K in staging vector `it` of slab k0.
@@ -644,13 +704,15 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     // `gm` = 0: a masked kernel's steady state, where every slab this one
     // stores or loads is unguarded and a next slab exists (see the loop
     // below), so the loads are unconditional and the compiler's waits exact.
-    // `gm` = 2: bounded loads; 3: and A's K tail cleared in the slab it stores;
-    // 4: and all but the newest load waited for before the first store.
+    // `gm` = 2: bounded loads; 4: and all but the newest load waited for before
+    // the first store; 3: nothing left to load, A's K tail cleared in the slab it
+    // stores (masked kernels); 5: the last slab, nothing to load or store.
     auto slab = [&](auto par, auto gm, int kt, auto bc) __attribute__((always_inline)) {
       constexpr int P = decltype(par)::value;
       constexpr int cur = P;
-      constexpr bool steady = decltype(gm)::value != 1, bounded = decltype(gm)::value >= 2;
-      const bool more = steady || kt + 1 < nk;
+      constexpr int mode = decltype(gm)::value;
+      constexpr bool steady = mode != 1 && mode != 5, bounded = mode == 2 || mode == 4;
+      const bool more = steady || (mode == 1 && kt + 1 < nk);
 #pragma unroll
       for (int kc = 0; kc < C; ++kc) {
         const int fs = kc & 1;
@@ -679,13 +741,13 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
                 constexpr int o = decltype(oc)::value;
                 if (o == op) {
                   if constexpr (o % 2 == 0) {
-                    if constexpr (o == 0 && decltype(gm)::value == 4) __builtin_amdgcn_s_waitcnt(0x0f71);  // vmcnt(1)
-                    if constexpr (decltype(gm)::value == 3)
+                    if constexpr (o == 0 && mode == 4) __builtin_amdgcn_s_waitcnt(0x0f71);  // vmcnt(1)
+                    if constexpr (mode == 3 && MASK)
                       clear_k_tail(std::integral_constant<int, SET>{}, std::integral_constant<int, o / 2>{}, (kt + 1) * BK);
                     store_item(std::integral_constant<int, SET>{}, std::integral_constant<int, o / 2>{}, cur ^ 1);
                   } else if constexpr (bounded) {
                     load_bounded(std::integral_constant<int, SET>{}, std::integral_constant<int, o / 2>{});
-                  } else {
+                  } else if constexpr (mode == 0) {
                     load_item(std::integral_constant<int, SET>{}, std::integral_constant<int, o / 2>{},
                               (kt + 1 + DEPTH) * BK);
                   }
@@ -742,10 +804,7 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
             load_slab(std::integral_constant<int, DEPTH == 2 ? (P ^ 1) : 0>{}, gm, (kt + 1 + DEPTH) * BK, bc);
         }
       }
-      if constexpr (bounded) {
-        off_a += BK * 4;
-        off_b += b_step;
-      }
+      if constexpr (bounded) at.template next<P>(a_step, b_step);
       // With an odd chunk count the next slab's first fragments landed in
       // slot 1; the loop expects them in slot 0.
       if constexpr (C % 2 == 1) {
@@ -795,61 +854,57 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
       if ((long)BM * lda + BK < kBufElems && 6L * BK * ldb + BN < kBufElems) {
         // Slab t is staged in register set t & 1.
         using Bounded = std::integral_constant<int, 2>;
-        using Last = std::integral_constant<int, MASK ? 3 : 2>;
+        using Closing = std::integral_constant<int, 3>;
+        using Final = std::integral_constant<int, 5>;
         using Set0 = std::integral_constant<int, 0>;
         using Set1 = std::integral_constant<int, 1>;
         const int a_elems = (MASK ? min(Mi - m0i, BM) : BM) * (int)lda - kbi;
         rsa = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, a_elems * 4, 0x00020000);
         bound_b(0);
-        auto load_all = [&](auto sc) __attribute__((always_inline)) {
-          static_for<NSTG>([&](auto qc) __attribute__((always_inline)) { load_bounded(sc, qc); });
-          off_a += BK * 4;
-          off_b += b_step;
-        };
-        load_all(Set0{});
-        load_all(Set1{});
-        stage_bias();
-        static_for<NSTG>([&](auto qc) __attribute__((always_inline)) {
-          if constexpr (MASK) clear_k_tail(Set0{}, qc, 0);
-          store_item(Set0{}, qc, 0);
-        });
-        load_all(Set0{});
-        __syncthreads();
-        load_frags(0, 0, 0);
         // B is walked in windows that 31-bit offsets reach: one unless this
-        // workgroup's K range of it exceeds 2 GiB.  From slab `end` on there is
-        // nothing left to load (A's resource is emptied: the next slabs would be
-        // real memory, the start of its next rows) and masked kernels store the K
-        // tail.
-        const int end = nk - 3;
+        // workgroup's K range of it exceeds 2 GiB.
         const int window = (Ki + 4L * BK) * ldb + BN < kBufElems ? nk : (int)((kBufElems - BN) / ((long)BK * ldb) - 4) & ~1;
-        int kt = 0;
-        auto steady = [&](auto mode, int stop) __attribute__((always_inline)) {
-          for (; kt < stop; kt += 2) {
-            slab(Set0{}, mode, kt, BufOn{});
-            slab(Set1{}, mode, kt + 1, BufOn{});
-          }
-        };
         // More workgroups than the four a CU holds: their loads crowd the memory
         // path, and waiting a slab earlier (the other workgroups compute
         // meanwhile) is faster: 4095x4097x1023 283 -> 277 us, against 280 with
         // guarded loads.  With fewer it only waits: 777x1111x333 10.0 -> 10.8.
         const bool crowded = G::CROWD && gx * gy > 4 * 256;
-        for (;;) {
-          const int stop = min(end, kt + window);
-          if constexpr (G::CROWD) {
-            if (crowded) steady(std::integral_constant<int, 4>{}, stop);
+        int kt = 0;
+        auto pairs = [&](auto mode, int stop) __attribute__((always_inline)) {
+          for (; kt < stop; kt += 2) {
+            slab(Set0{}, mode, kt, BufOn{});
+            slab(Set1{}, mode, kt + 1, BufOn{});
           }
-          if (!crowded) steady(Bounded{}, stop);
-          if (kt >= end) break;
-          bound_b((kt + 3) * BK);
-        }
-        rsa = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, 0, 0x00020000);
-        for (; kt + 1 < nk; kt += 2) {
-          slab(Set0{}, Last{}, kt, BufOn{});
-          slab(Set1{}, Last{}, kt + 1, BufOn{});
-        }
-        if (kt < nk) slab(Set0{}, Bounded{}, kt, BufOn{});
+        };
+        walk_slabs(
+            nk, window, kt,
+            [&](auto sc) __attribute__((always_inline)) {
+              static_for<NSTG>([&](auto qc) __attribute__((always_inline)) { load_bounded(sc, qc); });
+              at.template next<0>(a_step, b_step);
+            },
+            [&]() __attribute__((always_inline)) {
+              stage_bias();
+              static_for<NSTG>([&](auto qc) __attribute__((always_inline)) {
+                if constexpr (MASK) clear_k_tail(Set0{}, qc, 0);
+                store_item(Set0{}, qc, 0);
+              });
+            },
+            [&]() __attribute__((always_inline)) {
+              __syncthreads();
+              load_frags(0, 0, 0);
+            },
+            [&](int stop) __attribute__((always_inline)) {
+              if constexpr (G::CROWD) {
+                if (crowded) pairs(std::integral_constant<int, 4>{}, stop);
+              }
+              if (!crowded) pairs(Bounded{}, stop);
+            },
+            bound_b,
+            [&]() __attribute__((always_inline)) {
+              slab(Set0{}, Closing{}, kt, BufOn{});
+              slab(Set1{}, Closing{}, kt + 1, BufOn{});
+            },
+            [&]() __attribute__((always_inline)) { slab(Set0{}, Final{}, kt, BufOn{}); });
       } else {
         prologue();
         k_loop(BufOff{});
