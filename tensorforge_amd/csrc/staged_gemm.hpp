@@ -161,25 +161,29 @@ struct SlabOffsets {
 };
 
 // Walks nk slabs, kt being the next to compute (0 on entry): three loads ahead,
-// then pairs of slabs that load, in windows of `window` slabs of B, then at most
+// then pairs of slabs that load, in windows of window() slabs of B, then at most
 // three slabs that load nothing.
+//   rebase(t)    B's resource from slab t on
 //   load(set)    slabs 0, 1 and 2 into register sets 0, 1 and 0
 //   first()      slab 0 to LDS
 //   ready()      the barrier, and slab 0's first fragments
 //   steady(stop) slabs kt and kt + 1, each loading the slab three on, until kt >= stop
-//   rebase(t)    B's resource from slab t on
 //   pair(), last()  slabs kt and kt + 1; slab kt = nk - 1
-template <typename Load, typename First, typename Ready, typename Steady, typename Rebase, typename Pair, typename Last>
-__host__ __device__ __forceinline__ void walk_slabs(int nk, int window, int &kt, Load &&load, First &&first, Ready &&ready,
-                                                    Steady &&steady, Rebase &&rebase, Pair &&pair, Last &&last) {
+// (window() is asked for after the first loads: its 64-bit arithmetic before them made
+// a launch of a few slabs 5% slower.)
+template <typename Window, typename Rebase, typename Load, typename First, typename Ready, typename Steady, typename Pair,
+          typename Last>
+__host__ __device__ __forceinline__ void walk_slabs(int nk, int &kt, Window &&window, Rebase &&rebase, Load &&load,
+                                                    First &&first, Ready &&ready, Steady &&steady, Pair &&pair, Last &&last) {
+  rebase(0);
   load(std::integral_constant<int, 0>{});
   load(std::integral_constant<int, 1>{});
   first();
   load(std::integral_constant<int, 0>{});
   ready();
-  const int end = nk - 3;  // slab end - 1 loads slab nk - 1
+  const int end = nk - 3, win = window();  // slab end - 1 loads slab nk - 1
   for (;;) {
-    steady(end < kt + window ? end : kt + window);
+    steady(end < kt + win ? end : kt + win);
     if (kt >= end) break;
     rebase(kt + 3);
   }
@@ -860,10 +864,6 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
         using Set1 = std::integral_constant<int, 1>;
         const int a_elems = (MASK ? min(Mi - m0i, BM) : BM) * (int)lda - kbi;
         rsa = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, a_elems * 4, 0x00020000);
-        bound_b(0);
-        // B is walked in windows that 31-bit offsets reach: one unless this
-        // workgroup's K range of it exceeds 2 GiB.
-        const int window = (Ki + 4L * BK) * ldb + BN < kBufElems ? nk : (int)((kBufElems - BN) / ((long)BK * ldb) - 4) & ~1;
         // More workgroups than the four a CU holds: their loads crowd the memory
         // path, and waiting a slab earlier (the other workgroups compute
         // meanwhile) is faster: 4095x4097x1023 283 -> 277 us, against 280 with
@@ -877,7 +877,13 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
           }
         };
         walk_slabs(
-            nk, window, kt,
+            nk, kt,
+            // B is walked in windows that 31-bit offsets reach: one unless this
+            // workgroup's K range of it exceeds 2 GiB.
+            [&]() __attribute__((always_inline)) {
+              return (Ki + 4L * BK) * ldb + BN < kBufElems ? nk : (int)((kBufElems - BN) / ((long)BK * ldb) - 4) & ~1;
+            },
+            bound_b,
             [&](auto sc) __attribute__((always_inline)) {
               static_for<NSTG>([&](auto qc) __attribute__((always_inline)) { load_bounded(sc, qc); });
               at.template next<0>(a_step, b_step);
@@ -899,7 +905,6 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
               }
               if (!crowded) pairs(Bounded{}, stop);
             },
-            bound_b,
             [&]() __attribute__((always_inline)) {
               slab(Set0{}, Closing{}, kt, BufOn{});
               slab(Set1{}, Closing{}, kt + 1, BufOn{});

@@ -49,9 +49,8 @@ struct Model {
   bool run(int window) {
     int done = 0;
     size_a = 4L * (k - kb);
-    rebase(0);
     tfk::walk_slabs(
-        nk, window, kt,
+        nk, kt, [&]() { return window; }, [&](int first) { rebase(first); },
         [&](auto set) {
           load(decltype(set)::value);
           at.next<0>(a_step(), b_step());
@@ -64,7 +63,6 @@ struct Model {
             done += 2;
           }
         },
-        [&](int first) { rebase(first); },
         [&]() {
           slab<0>(kt, false, true);
           slab<1>(kt + 1, false, true);
