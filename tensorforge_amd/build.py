@@ -48,7 +48,7 @@ def _units():
     import gen_instances  # noqa: E402
     gen_instances.main()
     units = [CSRC / "runtime.hip", CSRC / "direct_kernels.hip", CSRC / "_gen" / "registry.hip",
-             CSRC / "_gen" / "wavek.hip", CSRC / "_gen" / "seq.hip"]
+             CSRC / "_gen" / "wavek.hip", CSRC / "_gen" / "forms.hip"]
     units += sorted((CSRC / "_gen").glob("staged_*.hip"))
     return units
 
@@ -96,12 +96,12 @@ def _demangle(names):
 def _entry_name(demangled):
     m = re.search(r"staged_gemm_kernel<(\d+), (\d+), (\d+), (\d+), (\d+), (\d+), (\d+), (\d+), (\d+)>", demangled)
     if m:
-        bm, bn, tm, tn, bk, p, v, mk, seq = m.groups()
-        if seq == "1":
+        bm, bn, tm, tn, bk, p, v, mk, form = m.groups()
+        if form == "1":
             import gen_instances  # noqa: E402  (csrc is on sys.path after _units)
             return gen_instances.seq_name(tuple(int(x) for x in (bm, bn, tm, tn, bk, mk)))
         return (f"tf_staged_b{bm}x{bn}_t{tm}x{tn}_k{bk}" + ("" if p == "1" else "_noprom") +
-                ("" if v == "1" else "_novec") + ("_masked" if mk == "1" else ""))
+                ("" if v == "1" else "_novec") + ("_masked" if mk == "1" else "") + ("_crowd" if form == "2" else ""))
     m = re.search(r"wavek_gemm_kernel<(\d+), (\d+), (\d+), (\d+)(?:, \d+)?>", demangled)
     if m:
         # One kernel serves every thread tile with its thread count.

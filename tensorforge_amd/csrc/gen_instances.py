@@ -205,6 +205,11 @@ def seq_name(c):
     return f"tf_seq_b{bm}x{bn}_t{tm}x{tn}_k{bk}" + ("_masked" if mk else "")
 
 
+# Crowded-grid forms (crowd_entry in runtime.hip) of this staged configuration and
+# its masked twin.
+CROWD_CONFIG = (64, 64, 4, 4, 16, 1, 1)
+
+
 def main(shards=16):
     gen = HERE / "_gen"
     gen.mkdir(exist_ok=True)
@@ -218,7 +223,7 @@ def main(shards=16):
             lines.append(f"    KernelEntry{{FAM_STAGED, {t}, \"{name(c)}\",")
             lines.append(f"                reinterpret_cast<const void *>(&staged_gemm_kernel<{t}>),")
             t7 = ", ".join(str(x) for x in c[:7])
-            lines.append(f"                &launch_staged<{t}>, nullptr, StagedGemm<{t7}, 0, {c[7]}>::LDS_BYTES}},")
+            lines.append(f"                &launch_staged<{t}>, nullptr, StagedGemm<{t7}>::LDS_BYTES}},")
         lines += ["};", f"extern const int kStagedCount{i} = {len(part)};", "#else",
                   "// Device pass: instantiate the kernels the host table names."]
         for c in part:
@@ -252,22 +257,24 @@ def main(shards=16):
     if not p.exists() or p.read_text() != text:
         p.write_text(text)
     seq = [c + (mk,) for c in SEQ_CONFIGS for mk in (0, 1)]
+    forms = [("FAM_DIRECT", "FORM_SEQ", c[:5] + (1, 1), c[5], seq_name(c)) for c in seq]
+    forms += [("FAM_STAGED", "FORM_CROWD", CROWD_CONFIG, mk, name(CROWD_CONFIG + (mk,)) + "_crowd") for mk in (0, 1)]
     lines = ['#include "../staged_gemm.hpp"', "", "namespace tfk {", "",
-             "#ifndef __HIP_DEVICE_COMPILE__  // host table", "extern const KernelEntry kSeqEntries[] = {"]
-    for c in seq:
-        bm, bn, tm, tn, bk, mk = c
-        t = f"{bm}, {bn}, {tm}, {tn}, {bk}, 1, 1"
-        lines.append(f"    KernelEntry{{FAM_DIRECT, {t}, {mk}, \"{seq_name(c)}\",")
-        lines.append(f"                reinterpret_cast<const void *>(&staged_gemm_kernel<{t}, {mk}, 1>),")
-        lines.append(f"                &launch_staged<{t}, {mk}, 1>, nullptr, StagedGemm<{t}, 1>::LDS_BYTES}},")
-    lines += ["};", f"extern const int kSeqCount = {len(seq)};", "#else",
+             "#ifndef __HIP_DEVICE_COMPILE__  // host table", "extern const KernelEntry kFormEntries[] = {"]
+    for fam, form, cfg, mk, nm in forms:
+        t = ", ".join(str(x) for x in cfg)
+        lines.append(f"    KernelEntry{{{fam}, {t}, {mk}, \"{nm}\",")
+        lines.append(f"                reinterpret_cast<const void *>(&staged_gemm_kernel<{t}, {mk}, {form}>),")
+        lines.append(f"                &launch_staged<{t}, {mk}, {form}>, nullptr, StagedGemm<{t}, {form}>::LDS_BYTES}},")
+    lines += ["};", f"extern const int kFormCount = {len(forms)};", "#else",
               "// Device pass: instantiate the kernels the host table names."]
-    for bm, bn, tm, tn, bk, mk in seq:
-        lines.append(f"template __global__ void staged_gemm_kernel<{bm}, {bn}, {tm}, {tn}, {bk}, 1, 1, {mk}, 1>(const float *, "
+    for _, form, cfg, mk, _ in forms:
+        t = ", ".join(str(x) for x in cfg)
+        lines.append(f"template __global__ void staged_gemm_kernel<{t}, {mk}, {form}>(const float *, "
                      "const float *, long, long, int, int, int, int, int, int, GemmParams);")
     lines += ["#endif", "", "}  // namespace tfk", ""]
     text = "\n".join(lines)
-    p = gen / "seq.hip"
+    p = gen / "forms.hip"
     if not p.exists() or p.read_text() != text:
         p.write_text(text)
     reg = ['#include <vector>', '', '#include "../tf_kernels.h"', '', 'namespace tfk {', '',

@@ -116,11 +116,11 @@ void staged_wave_layout(long bm, long bn, long tm, long tn, long &ktm, long &ktn
 struct Launch {
   const tfk::KernelEntry *entry = nullptr;
   dim3 grid, block;
-  // Direct GEMMs: the matrix-core form of the same arithmetic that runs
-  // instead wherever every buffer is 16-byte aligned (seq_entry), with its own
-  // geometry; null where the problem has none.
-  const tfk::KernelEntry *seq = nullptr;
-  dim3 seq_grid, seq_block;
+  // Another form of the same arithmetic that runs instead where every buffer is
+  // 16-byte aligned, with its own geometry: direct GEMMs on the matrix cores
+  // (seq_entry), staged ones on crowded grids (crowd_entry); null where there is none.
+  const tfk::KernelEntry *form = nullptr;
+  dim3 form_grid, form_block;
 };
 
 long ceil_div(long a, long b) { return (a + b - 1) / b; }
@@ -155,14 +155,32 @@ const tfk::KernelEntry *seq_entry(long M, long N, long K) {
     const double time = t.start + rounds * K * (t.cost + (ragged(t.edge) ? t.cost / 12 : 0));
     if (!best || time < best_time) best = &t, best_time = time;
   }
-  for (int i = 0; i < tfk::kSeqCount; ++i) {
-    const tfk::KernelEntry &e = tfk::kSeqEntries[i];
+  for (int i = 0; i < tfk::kFormCount; ++i) {
+    const tfk::KernelEntry &e = tfk::kFormEntries[i];
+    if (e.family != tfk::FAM_DIRECT) continue;
     if (e.bm != best->edge || (e.bm == 32 && e.bk != small_k()) || e.masked != ragged(e.bm)) continue;
     // The kernels number the tiles in 32 bits; masked twins index A and B with
     // 32-bit offsets (tiles may run one block past the edges).
     if (ceil_div(M, e.bm) * ceil_div(N, e.bn) >= (1L << 31)) return nullptr;
     if (e.masked && ((M + 256) * K >= (1L << 31) || (K + 64) * (N + 256) >= (1L << 31))) return nullptr;
     return &e;
+  }
+  return nullptr;
+}
+
+// The crowded-grid form of staged entry `e` (StagedGemm::CROWD), or null: none, or
+// the grid has no more workgroups than its plain form runs at once, six per CU.
+// Both sides, us, plain / crowded: unmasked 2048x2048x1024 (1024 workgroups) 68.6 /
+// 68.7, 2112x2112x704 (1089) 58.9 / 59.9, 2560x2560x512 (1600) 61.7 / 61.6,
+// 2112x3328x704 (1716) 92.0 / 82.3; masked 2100x2100x700 (1089) 63.1 / 64.9,
+// 2100x3300x700 (1716) 91.7 / 85.9.
+const tfk::KernelEntry *crowd_entry(const tfk::KernelEntry &e, dim3 grid) {
+  if ((long)grid.x * grid.y * grid.z <= 6 * 256) return nullptr;
+  for (int i = 0; i < tfk::kFormCount; ++i) {
+    const tfk::KernelEntry &f = tfk::kFormEntries[i];
+    if (f.family == tfk::FAM_STAGED && e.family == f.family && f.bm == e.bm && f.bn == e.bn && f.tm == e.tm &&
+        f.tn == e.tn && f.bk == e.bk && f.promote == e.promote && f.vectorize == e.vectorize && f.masked == e.masked)
+      return &f;
   }
   return nullptr;
 }
@@ -281,10 +299,10 @@ int select_launches(tf_kernel *k) {
     L.block = dim3((unsigned)tx, (unsigned)ty, 1);
     L.grid = dim3((unsigned)std::max(1L, ceil_div(st.N, o.bn)), (unsigned)std::max(1L, ceil_div(st.M, o.bm)), 1);
     if (gemm && !staged && st.M > 0 && st.N > 0) {
-      L.seq = seq_entry(st.M, st.N, st.K);
-      if (L.seq) {
-        L.seq_block = dim3((unsigned)(L.seq->bn / L.seq->tn), (unsigned)(L.seq->bm / L.seq->tm), 1);
-        L.seq_grid = dim3((unsigned)ceil_div(st.N, L.seq->bn), (unsigned)ceil_div(st.M, L.seq->bm), 1);
+      L.form = seq_entry(st.M, st.N, st.K);
+      if (L.form) {
+        L.form_block = dim3((unsigned)(L.form->bn / L.form->tn), (unsigned)(L.form->bm / L.form->tm), 1);
+        L.form_grid = dim3((unsigned)ceil_div(st.N, L.form->bn), (unsigned)ceil_div(st.M, L.form->bm), 1);
       }
     }
     // split-k splits the K loop of GEMM stages; the element-op launches of an
@@ -302,6 +320,11 @@ int select_launches(tf_kernel *k) {
       L.grid.z = (unsigned)o.split_k;
       // Whole tiles per slice: (grid.y * BM) x (grid.x * BN).
       k->ws_bytes = std::max(k->ws_bytes, (size_t)o.split_k * L.grid.y * o.bm * L.grid.x * o.bn * sizeof(float));
+    }
+    if (staged && !wavek) {
+      L.form = crowd_entry(*L.entry, L.grid);
+      L.form_grid = L.grid;
+      L.form_block = L.block;
     }
     k->launches.push_back(L);
   }
@@ -327,16 +350,17 @@ int launch_stage(const tf_kernel *k, size_t s, void *const *ptrs, void *ws, hipS
   if (st.M == 0 || st.N == 0) return TF_OK;
   // 128-bit accesses need 16-byte aligned buffers (the reference's ABI
   // guarantees 256-byte alignment: docs/stage8.md:34).
-  bool use_seq = L.seq != nullptr;
-  if (use_seq || L.entry->family == tfk::FAM_STAGED || L.entry->family == tfk::FAM_WAVEK) {
+  bool use_form = L.form != nullptr;
+  if (use_form || L.entry->family == tfk::FAM_STAGED || L.entry->family == tfk::FAM_WAVEK) {
     std::vector<int> ids = {st.a, st.b, st.out};
     for (const tff::EpiOp &e : st.epi)
       if (e.buf >= 0) ids.push_back(e.buf);
     for (int id : ids)
       if (reinterpret_cast<uintptr_t>(ptrs[id]) % 16 != 0) {
         // The direct kernel takes any alignment.
-        if (!use_seq) return fail(TF_E_ARG, "buffer " + std::to_string(id) + " is not 16-byte aligned");
-        use_seq = false;
+        if (L.entry->family != tfk::FAM_DIRECT)
+          return fail(TF_E_ARG, "buffer " + std::to_string(id) + " is not 16-byte aligned");
+        use_form = false;
         break;
       }
   }
@@ -360,7 +384,7 @@ int launch_stage(const tf_kernel *k, size_t s, void *const *ptrs, void *ws, hipS
       p.ws_ld = (long)L.grid.x * L.entry->bn;
       p.ws_slice = p.ws_ld * L.grid.y * L.entry->bm;
     }
-    err = use_seq ? L.seq->gemm(p, L.seq_grid, L.seq_block, stream) : L.entry->gemm(p, L.grid, L.block, stream);
+    err = use_form ? L.form->gemm(p, L.form_grid, L.form_block, stream) : L.entry->gemm(p, L.grid, L.block, stream);
     if (err == hipSuccess && p.splits > 1) {
       tfk::ReduceParams r{};
       r.ws = p.ws;

@@ -198,8 +198,13 @@ __host__ __device__ __forceinline__ void walk_slabs(int nk, int &kt, Window &&wi
 __device__ __forceinline__ void put(float &v, int, float x) { v = x; }
 __device__ __forceinline__ void put(f32x4 &v, int e, float x) { v[e] = x; }
 
-template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC, int SEQ = 0, int MASK = 0>
+// Forms of the staged kernel: the plain one; sequential k; and, for grids of more
+// workgroups than its plain form runs at once, the crowded one (see CROWD).
+enum Form : int { FORM_PLAIN = 0, FORM_SEQ = 1, FORM_CROWD = 2 };
+
+template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC, int FORM = FORM_PLAIN>
 struct StagedGemm {
+  static constexpr int SEQ = FORM == FORM_SEQ;
   static constexpr int NT = (BM / TM) * (BN / TN);
   static constexpr int WTM = 8 * TM, WTN = 8 * TN;
   static constexpr int NWM = BM / WTM, NWN = BN / WTN;
@@ -221,10 +226,19 @@ struct StagedGemm {
   static constexpr int B_ROW_G = SEQ ? 1 : 4, B_ROW_S = SEQ ? 64 / MB : 1;
   static constexpr int A_ELEMS = BM * LDA, B_ELEMS = BK * LDB;
   // Two A and B tile buffers, plus the tile's BN bias values.
-  // Masked 64x64 t4x4 k16 (CROWD): padded to four workgroups per CU.  A slab is
-  // half of each 128-byte line of its A rows; six workgroups' lines outlive
-  // the L1 before the next slab wants the other half.
-  static constexpr bool CROWD = MASK && !SEQ && PROMOTE && VEC && BM == 64 && BN == 64 && TM == 4 && TN == 4 && BK == 16;
+  // Crowded grids (64x64 t4x4 k16, chosen by crowd_entry in runtime.hip).  A slab is
+  // half of each 128-byte line of its A rows, and the plain form's five or six
+  // workgroups per CU keep more lines in flight than outlive the L1 until the next
+  // slab wants the other half: padded to four per CU.  And a branch to the next
+  // instruction before a slab's first LDS write: it empties the wave's instruction
+  // buffer, and waves that meet at their writes drift apart.  (Found by timing: 16
+  // idle cycles there are slower on small grids and no better on large ones, s_sleep
+  // 0 does nothing, waiting for all but the newest load does half of it.)  us, plain /
+  // padded / padded with the branch: unmasked 2112x3328x704 92.0 / 82.6 / 82.3,
+  // 3008x3008x1008 156.6 / 158.3 / 146.9, 4096x4096x1024 275.9 / 275.8 / 262.7; masked
+  // 2600x2900x1200 165.4 / 155.6 / 155.6, 3000x3000x1000 158.7 / 160.0 / 149.0,
+  // 4095x4097x1023 291.7 / 291.1 / 287.5.
+  static constexpr int CROWD = FORM == FORM_CROWD;
   static constexpr int CROWD_PAD = CROWD ? 13312 / 4 : 0;
   static constexpr int LDS_BYTES = PROMOTE ? 2 * (A_ELEMS + B_ELEMS) * 4 + (BN + CROWD_PAD) * 4 : 0;
   // Global -> register staging per thread and slab.
@@ -287,7 +301,7 @@ struct StagedGemm {
 // by-value struct is read from the kernel-argument segment (a ~1.5k-cycle
 // round trip measured at the start of every wave).  gx, gy = gridDim.x, .y;
 // flags = swizzle | splits << 8.
-template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC, int MASK, int SEQ = 0>
+template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC, int MASK, int FORM = FORM_PLAIN>
 __global__ void __launch_bounds__((BM / TM) * (BN / TN))
 staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int pK, int gx, int gy, int flags, int pM,
                    int pN, GemmParams p) {
@@ -300,7 +314,8 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
   p.N = pN;
   p.swizzle = flags & 255;
   p.splits = flags >> 8;
-  using G = StagedGemm<BM, BN, TM, TN, BK, PROMOTE, VEC, SEQ, MASK>;
+  using G = StagedGemm<BM, BN, TM, TN, BK, PROMOTE, VEC, FORM>;
+  constexpr bool SEQ = G::SEQ;
   constexpr int NT = G::NT, WTM = G::WTM, WTN = G::WTN, NWN = G::NWN, FM = G::FM, FN = G::FN;
   constexpr int LDA = G::LDA, LDB = G::LDB, VW = G::VW, MB = G::MB, KC = G::KC;
   using AccT = AccOf<MB>;
@@ -708,14 +723,13 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     // `gm` = 0: a masked kernel's steady state, where every slab this one
     // stores or loads is unguarded and a next slab exists (see the loop
     // below), so the loads are unconditional and the compiler's waits exact.
-    // `gm` = 2: bounded loads; 4: and all but the newest load waited for before
-    // the first store; 3: nothing left to load, A's K tail cleared in the slab it
-    // stores (masked kernels); 5: the last slab, nothing to load or store.
+    // `gm` = 2: bounded loads; 3: nothing left to load, A's K tail cleared in the
+    // slab it stores (masked kernels); 4: the last slab, nothing to load or store.
     auto slab = [&](auto par, auto gm, int kt, auto bc) __attribute__((always_inline)) {
       constexpr int P = decltype(par)::value;
       constexpr int cur = P;
       constexpr int mode = decltype(gm)::value;
-      constexpr bool steady = mode != 1 && mode != 5, bounded = mode == 2 || mode == 4;
+      constexpr bool steady = mode != 1 && mode != 4, bounded = mode == 2;
       const bool more = steady || (mode == 1 && kt + 1 < nk);
 #pragma unroll
       for (int kc = 0; kc < C; ++kc) {
@@ -745,7 +759,7 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
                 constexpr int o = decltype(oc)::value;
                 if (o == op) {
                   if constexpr (o % 2 == 0) {
-                    if constexpr (o == 0 && mode == 4) __builtin_amdgcn_s_waitcnt(0x0f71);  // vmcnt(1)
+                    if constexpr (o == 0 && bounded && G::CROWD) asm volatile("s_branch 0");  // to the next instruction
                     if constexpr (mode == 3 && MASK)
                       clear_k_tail(std::integral_constant<int, SET>{}, std::integral_constant<int, o / 2>{}, (kt + 1) * BK);
                     store_item(std::integral_constant<int, SET>{}, std::integral_constant<int, o / 2>{}, cur ^ 1);
@@ -859,23 +873,12 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
         // Slab t is staged in register set t & 1.
         using Bounded = std::integral_constant<int, 2>;
         using Closing = std::integral_constant<int, 3>;
-        using Final = std::integral_constant<int, 5>;
+        using Final = std::integral_constant<int, 4>;
         using Set0 = std::integral_constant<int, 0>;
         using Set1 = std::integral_constant<int, 1>;
         const int a_elems = (MASK ? min(Mi - m0i, BM) : BM) * (int)lda - kbi;
         rsa = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, a_elems * 4, 0x00020000);
-        // More workgroups than the four a CU holds: their loads crowd the memory
-        // path, and waiting a slab earlier (the other workgroups compute
-        // meanwhile) is faster: 4095x4097x1023 283 -> 277 us, against 280 with
-        // guarded loads.  With fewer it only waits: 777x1111x333 10.0 -> 10.8.
-        const bool crowded = G::CROWD && gx * gy > 4 * 256;
         int kt = 0;
-        auto pairs = [&](auto mode, int stop) __attribute__((always_inline)) {
-          for (; kt < stop; kt += 2) {
-            slab(Set0{}, mode, kt, BufOn{});
-            slab(Set1{}, mode, kt + 1, BufOn{});
-          }
-        };
         walk_slabs(
             nk, kt,
             // B is walked in windows that 31-bit offsets reach: one unless this
@@ -900,10 +903,10 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
               load_frags(0, 0, 0);
             },
             [&](int stop) __attribute__((always_inline)) {
-              if constexpr (G::CROWD) {
-                if (crowded) pairs(std::integral_constant<int, 4>{}, stop);
+              for (; kt < stop; kt += 2) {
+                slab(Set0{}, Bounded{}, kt, BufOn{});
+                slab(Set1{}, Bounded{}, kt + 1, BufOn{});
               }
-              if (!crowded) pairs(Bounded{}, stop);
             },
             [&]() __attribute__((always_inline)) {
               slab(Set0{}, Closing{}, kt, BufOn{});
@@ -1043,10 +1046,10 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
   }
 }
 
-template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC, int MASK, int SEQ = 0>
+template <int BM, int BN, int TM, int TN, int BK, int PROMOTE, int VEC, int MASK, int FORM = FORM_PLAIN>
 hipError_t launch_staged(const GemmParams &p, dim3 grid, dim3 block, hipStream_t stream) {
   if (block.x != BN / TN || block.y != BM / TM || block.z != 1) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((staged_gemm_kernel<BM, BN, TM, TN, BK, PROMOTE, VEC, MASK, SEQ>), grid, block, 0, stream, p.A, p.B,
+  hipLaunchKernelGGL((staged_gemm_kernel<BM, BN, TM, TN, BK, PROMOTE, VEC, MASK, FORM>), grid, block, 0, stream, p.A, p.B,
                      p.lda, p.ldb, p.K, (int)grid.x, (int)grid.y, p.swizzle | (p.splits << 8), p.M, p.N, p);
   return hipGetLastError();
 }

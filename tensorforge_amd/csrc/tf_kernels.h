@@ -89,10 +89,12 @@ hipError_t launch_elementwise_flat(const EltParams &p, hipStream_t stream);
 // The split-K reduction (direct_kernels.hip); ws and C 16-byte aligned.
 hipError_t launch_splitk_reduce(const ReduceParams &p, hipStream_t stream);
 
-// The sequential-k staged instantiations (generated _gen/seq.hip): the
-// matrix-core form of the direct kernel, each followed by its masked twin.
-extern const KernelEntry kSeqEntries[];
-extern const int kSeqCount;
+// Other forms of the staged kernel (generated _gen/forms.hip), chosen by the runtime
+// from the problem's size and each followed by its masked twin: sequential k, the
+// matrix-core form of the direct kernel (family FAM_DIRECT), and the form for
+// crowded grids (FAM_STAGED).
+extern const KernelEntry kFormEntries[];
+extern const int kFormCount;
 
 // Registry (defined in the generated registry translation unit).
 const KernelEntry *registry_begin();
