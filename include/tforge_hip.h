@@ -38,9 +38,6 @@ extern "C" {
 #define TF_E_BLAS -6     /* vendor BLAS baseline unavailable or failed        */
 
 #define TF_FAMILY_DIRECT 0      /* tile-k=0: one FMA chain per output          */
-/* (A TF_FAMILY_DIRECT launch reports the options' own geometry.  On 16-byte
- * aligned buffers its chains run on the matrix cores, in workgroups the library
- * sizes to the problem; the result is the same bits.) */
 #define TF_FAMILY_STAGED 1      /* tile-k>0: LDS-staged FP32 MFMA              */
 #define TF_FAMILY_ELEMENTWISE 2 /* programs without a matmul                   */
 #define TF_FAMILY_WAVEK 4       /* tile-k>0 with wave-split-k: the waves of a
@@ -148,6 +145,14 @@ void tf_kernel_free(tf_kernel_t *k);
  * runners/gpu/tforge-gpu-bench.cu:20-24, 92-140). */
 int tf_kernel_num_launches(const tf_kernel_t *k);
 int tf_kernel_launch_info(const tf_kernel_t *k, int launch, tf_launch_info_t *out);
+/* tf_kernel_launch_info describes the options' own kernel; this one the kernel that
+ * runs where every buffer is 16-byte aligned, chosen by the problem's size with the
+ * same results bit for bit: a direct GEMM's chains on the matrix cores, element ops
+ * as one stream of vectors, a staged kernel's form for crowded grids, or the options'
+ * own.  On other buffers direct GEMMs and element ops run the options' own kernel and
+ * staged ones are refused.  No counterpart in the reference, which launches the kernel
+ * it generated. */
+int tf_kernel_run_info(const tf_kernel_t *k, int launch, tf_launch_info_t *out);
 int tf_kernel_num_buffers(const tf_kernel_t *k); /* entry arguments + 1 result */
 int tf_kernel_buffer_info(const tf_kernel_t *k, int index, tf_buffer_info_t *out);
 /* Shape (rows x cols) of buffer `index` as tf_run / tf_bench copy it from and
@@ -160,8 +165,8 @@ int tf_kernel_buffer_info(const tf_kernel_t *k, int index, tf_buffer_info_t *out
  * runner's per-buffer --in-dir file sizes (runners/gpu/tforge-gpu-bench.cu:214-232). */
 int tf_kernel_host_shape(const tf_kernel_t *k, const long long *logical_mnk, int index, long long *rows,
                          long long *cols);
-/* Resources and occupancy of one launch: the runner's --info-only
- * (runners/gpu/tforge-gpu-bench.cu:278-291). */
+/* Resources and occupancy of one launch's kernel (tf_kernel_run_info's): the
+ * runner's --info-only (runners/gpu/tforge-gpu-bench.cu:278-291). */
 int tf_kernel_info(const tf_kernel_t *k, int launch, tf_kernel_resources_t *out);
 
 /* Kernel ABI: enqueue every launch of the program on `stream` (a hipStream_t,

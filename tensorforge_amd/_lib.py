@@ -58,6 +58,7 @@ SIGNATURES = [
     ("tf_kernel_free", None, [P]),
     ("tf_kernel_num_launches", I, [P]),
     ("tf_kernel_launch_info", I, [P, I, ctypes.POINTER(LaunchInfo)]),
+    ("tf_kernel_run_info", I, [P, I, ctypes.POINTER(LaunchInfo)]),
     ("tf_kernel_num_buffers", I, [P]),
     ("tf_kernel_buffer_info", I, [P, I, ctypes.POINTER(BufferInfo)]),
     ("tf_kernel_host_shape", I, [P, ctypes.POINTER(LL), I, ctypes.POINTER(LL), ctypes.POINTER(LL)]),
@@ -135,10 +136,15 @@ class Kernel:
         for i in range(check(L.tf_kernel_num_launches(self.h))):
             li = LaunchInfo()
             check(L.tf_kernel_launch_info(self.h, i, ctypes.byref(li)))
+            run = LaunchInfo()
+            check(L.tf_kernel_run_info(self.h, i, ctypes.byref(run)))
             out.append({"kernel": li.kernel.decode(), "grid": list(li.grid), "block": list(li.block),
                         "args": li.args.decode().split(","), "ops": li.ops.decode(),
                         "family": FAMILY_NAMES[li.family], "m": li.m, "n": li.n, "k": li.k,
-                        "lds_bytes": li.lds_bytes})
+                        "lds_bytes": li.lds_bytes,
+                        # what runs on 16-byte aligned buffers
+                        "run": {"kernel": run.kernel.decode(), "grid": list(run.grid), "block": list(run.block),
+                                "lds_bytes": run.lds_bytes}})
         return out
 
     def buffers(self):

@@ -108,6 +108,10 @@ def _entry_name(demangled):
         import gen_instances  # noqa: E402  (csrc is on sys.path after _units)
         bm, bn, nt, bk = (int(x) for x in m.groups())
         return [gen_instances.wavek_name(bm, bn, tm, tn, bk) for tm, tn in gen_instances.wavek_thread_tiles(bm, bn, nt)]
+    m = re.search(r"elementwise_flat_kernel<unsigned (int|long), (\w+), (\d+)u, (\d+)u>", demangled)
+    if m:
+        idx = "uint32_t" if m.group(1) == "int" else "uint64_t"
+        return f"tf_elementwise_flat_{idx}_{m.group(2)}_w{m.group(3)}s{m.group(4)}"
     m = re.search(r"(direct_gemm|elementwise)_kernel<(\d+), (\d+)>", demangled)
     if m:
         fam = "direct" if m.group(1) == "direct_gemm" else "elementwise"

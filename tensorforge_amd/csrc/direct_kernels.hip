@@ -191,32 +191,54 @@ hipError_t launch_elementwise(const EltParams &p, dim3 grid, dim3 block, hipStre
   return hipGetLastError();
 }
 
-template <typename Idx, unsigned WAVES, unsigned SEG>
-static hipError_t launch_flat(const EltParams &p, const float *bias, const float *r, unsigned kinds, bool one,
-                              hipStream_t stream) {
-  const long total = (long)p.M * p.N, span = 64 * WAVES * SEG;
-  const long groups = std::max(1L, (total / 4 + span - 1) / span * SEG);
-  const unsigned n = (unsigned)p.N, inv = n > 1 ? (unsigned)((1UL << 32) / n) : ~0u;
-  auto fn = one ? &elementwise_flat_kernel<Idx, true, WAVES, SEG> : &elementwise_flat_kernel<Idx, false, WAVES, SEG>;
-  hipLaunchKernelGGL(fn, dim3((unsigned)std::min(groups, kMaxFlatGrid)), dim3(64 * WAVES), 0, stream, p.X, p.Y, total, bias,
-                     r, n, inv, kinds, p);
-  return hipGetLastError();
+using FlatFn = void (*)(const float *, float *, long, const float *, const float *, unsigned, unsigned, unsigned, EltParams);
+struct FlatKernel {
+  const char *name;
+  FlatFn fn;
+  unsigned waves, seg;
+};
+
+static int count_kind(const EltParams &p, int kind) {
+  int n = 0;
+  for (int i = 0; i < p.epi.nops; ++i) n += p.epi.kind[i] == kind;
+  return n;
+}
+
+#define TF_FLAT(IDX, ONE, WAVES, SEG) \
+  FlatKernel{"tf_elementwise_flat_" #IDX "_" #ONE "_w" #WAVES "s" #SEG, &elementwise_flat_kernel<IDX, ONE, WAVES, SEG>, WAVES, SEG}
+static const FlatKernel &flat_kernel(const EltParams &p) {
+  static const FlatKernel kFlat[3][2] = {{TF_FLAT(uint32_t, false, 8, 32), TF_FLAT(uint32_t, true, 8, 32)},
+                                         {TF_FLAT(uint32_t, false, 4, 4), TF_FLAT(uint32_t, true, 4, 4)},
+                                         {TF_FLAT(uint64_t, false, 4, 4), TF_FLAT(uint64_t, true, 4, 4)}};
+  const long total = (long)p.M * p.N;
+  const bool one = count_kind(p, EPI_BIAS) <= 1 && count_kind(p, EPI_ADD) <= 1;
+  return kFlat[total < kHugeStream ? 0 : total < (1L << 32) ? 1 : 2][one];
+}
+#undef TF_FLAT
+
+static dim3 flat_grid(const EltParams &p, const FlatKernel &k) {
+  const long vecs = (long)p.M * p.N / 4, span = 64 * k.waves * k.seg;
+  return dim3((unsigned)std::min(std::max(1L, (vecs + span - 1) / span * k.seg), kMaxFlatGrid));
+}
+
+FlatLaunch elementwise_flat_launch(const EltParams &p) {
+  const FlatKernel &k = flat_kernel(p);
+  return {k.name, reinterpret_cast<const void *>(k.fn), flat_grid(p, k), dim3(64 * k.waves)};
 }
 
 hipError_t launch_elementwise_flat(const EltParams &p, hipStream_t stream) {
   unsigned kinds = 0;
-  int biases = 0, adds = 0;
   const float *bias = nullptr, *r = nullptr;
   for (int i = 0; i < p.epi.nops; ++i) {
     kinds |= (unsigned)p.epi.kind[i] << (8 * i);
-    if (p.epi.kind[i] == EPI_BIAS) bias = p.epi.ptr[i], ++biases;
-    if (p.epi.kind[i] == EPI_ADD) r = p.epi.ptr[i], ++adds;
+    if (p.epi.kind[i] == EPI_BIAS) bias = p.epi.ptr[i];
+    if (p.epi.kind[i] == EPI_ADD) r = p.epi.ptr[i];
   }
-  const long total = (long)p.M * p.N;
-  const bool one = biases <= 1 && adds <= 1;
-  if (total < kHugeStream) return launch_flat<unsigned, 8, 32>(p, bias, r, kinds, one, stream);
-  if (total < (1L << 32)) return launch_flat<unsigned, 4, 4>(p, bias, r, kinds, one, stream);
-  return launch_flat<unsigned long, 4, 4>(p, bias, r, kinds, one, stream);
+  const FlatKernel &k = flat_kernel(p);
+  const unsigned n = (unsigned)p.N, inv = n > 1 ? (unsigned)((1UL << 32) / n) : ~0u;
+  hipLaunchKernelGGL(k.fn, flat_grid(p, k), dim3(64 * k.waves), 0, stream, p.X, p.Y, (long)p.M * p.N, bias, r, n, inv, kinds,
+                     p);
+  return hipGetLastError();
 }
 
 // Split-K reduction: one thread per 4 consecutive outputs; the partial-sum

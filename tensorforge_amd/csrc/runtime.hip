@@ -121,6 +121,9 @@ struct Launch {
   // (seq_entry), staged ones on crowded grids (crowd_entry); null where there is none.
   const tfk::KernelEntry *form = nullptr;
   dim3 form_grid, form_block;
+  // What runs on 16-byte aligned buffers: `form`, the flat kernel (element ops), or `entry`.
+  tfk::FlatLaunch run;
+  int run_lds;
 };
 
 long ceil_div(long a, long b) { return (a + b - 1) / b; }
@@ -326,6 +329,19 @@ int select_launches(tf_kernel *k) {
       L.form_grid = L.grid;
       L.form_block = L.block;
     }
+    if (gemm) {
+      const tfk::KernelEntry &e = L.form ? *L.form : *L.entry;
+      L.run = {e.name, e.fn, L.form ? L.form_grid : L.grid, L.form ? L.form_block : L.block};
+      L.run_lds = e.lds_bytes;
+    } else {
+      tfk::EltParams p{};
+      p.M = (int)st.M;
+      p.N = (int)st.N;
+      p.epi.nops = (int)st.epi.size();
+      for (int i = 0; i < p.epi.nops; ++i) p.epi.kind[i] = st.epi[i].kind;
+      L.run = tfk::elementwise_flat_launch(p);
+      L.run_lds = 0;
+    }
     k->launches.push_back(L);
   }
   return TF_OK;
@@ -365,6 +381,7 @@ int launch_stage(const tf_kernel *k, size_t s, void *const *ptrs, void *ws, hipS
       }
   }
   hipError_t err;
+  bool own = L.form && !use_form;  // the options' own kernel instead of L.run
   if (st.kind == tff::STAGE_GEMM) {
     tfk::GemmParams p{};
     p.A = static_cast<const float *>(ptrs[st.a]);
@@ -413,10 +430,12 @@ int launch_stage(const tf_kernel *k, size_t s, void *const *ptrs, void *ws, hipS
     bool flat = aligned(p.X) && aligned(p.Y);
     for (int i = 0; i < p.epi.nops; ++i)
       if (p.epi.kind[i] == tfk::EPI_ADD) flat = flat && aligned(p.epi.ptr[i]);
+    own = !flat;
     err = flat ? tfk::launch_elementwise_flat(p, stream) : L.entry->elt(p, L.grid, L.block, stream);
   }
   if (err != hipSuccess)
-    return fail(TF_E_HIP, std::string("kernel launch ") + L.entry->name + " failed: " + hipGetErrorString(err));
+    return fail(TF_E_HIP, std::string("kernel launch ") + (own ? L.entry->name : L.run.name) + " failed: " +
+                              hipGetErrorString(err));
   return TF_OK;
 }
 
@@ -840,6 +859,9 @@ static int compile_impl(const char *source_name, const char *program, const char
       std::fprintf(stderr, "// tforge-gpu: launch %zu: %s -> %s grid [%u, %u, 1] block [%u, %u, 1] M=%lld N=%lld K=%lld\n",
                    s, st.ops.c_str(), L.entry->name, L.grid.x, L.grid.y, L.block.x, L.block.y, (long long)st.M,
                    (long long)st.N, (long long)st.K);
+      if (L.run.fn != L.entry->fn)
+        std::fprintf(stderr, "// tforge-gpu:   on 16-byte aligned buffers: %s grid [%u, %u, %u] block [%u, %u, 1]\n",
+                     L.run.name, L.run.grid.x, L.run.grid.y, L.run.grid.z, L.run.block.x, L.run.block.y);
     }
   }
   *out = k.release();
@@ -883,6 +905,21 @@ int tf_kernel_launch_info(const tf_kernel_t *k, int launch, tf_launch_info_t *ou
   return TF_OK;
 }
 
+int tf_kernel_run_info(const tf_kernel_t *k, int launch, tf_launch_info_t *out) {
+  int rc = tf_kernel_launch_info(k, launch, out);
+  if (rc) return rc;
+  const Launch &L = k->launches[launch];
+  copy_str(out->kernel, sizeof(out->kernel), L.run.name);
+  out->grid[0] = L.run.grid.x;
+  out->grid[1] = L.run.grid.y;
+  out->grid[2] = L.run.grid.z;
+  out->block[0] = L.run.block.x;
+  out->block[1] = L.run.block.y;
+  out->block[2] = L.run.block.z;
+  out->lds_bytes = L.run_lds;
+  return TF_OK;
+}
+
 int tf_kernel_num_buffers(const tf_kernel_t *k) { return k ? k->plan.nargs + 1 : fail(TF_E_ARG, "null kernel"); }
 
 int tf_kernel_buffer_info(const tf_kernel_t *k, int index, tf_buffer_info_t *out) {
@@ -902,10 +939,10 @@ int tf_kernel_info(const tf_kernel_t *k, int launch, tf_kernel_resources_t *out)
   if (!k || !out || launch < 0 || launch >= (int)k->launches.size()) return fail(TF_E_ARG, "bad launch index");
   const Launch &L = k->launches[launch];
   hipFuncAttributes attr;
-  TF_HIP(hipFuncGetAttributes(&attr, L.entry->fn));
-  const int threads = (int)(L.block.x * L.block.y * L.block.z);
+  TF_HIP(hipFuncGetAttributes(&attr, L.run.fn));
+  const int threads = (int)(L.run.block.x * L.run.block.y * L.run.block.z);
   int blocks = 0;
-  TF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, L.entry->fn, threads, 0));
+  TF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, L.run.fn, threads, 0));
   hipDeviceProp_t prop;
   TF_HIP(hipGetDeviceProperties(&prop, 0));
   std::memset(out, 0, sizeof(*out));

@@ -86,6 +86,15 @@ struct KernelEntry {
 // 16-byte aligned, biases at any alignment (direct_kernels.hip).
 hipError_t launch_elementwise_flat(const EltParams &p, hipStream_t stream);
 
+// The instantiation that launch_elementwise_flat runs for p's sizes and ops (its
+// pointers are not looked at), and its geometry.
+struct FlatLaunch {
+  const char *name;
+  const void *fn;
+  dim3 grid, block;
+};
+FlatLaunch elementwise_flat_launch(const EltParams &p);
+
 // The split-K reduction (direct_kernels.hip); ws and C 16-byte aligned.
 hipError_t launch_splitk_reduce(const ReduceParams &p, hipStream_t stream);
 

@@ -238,7 +238,7 @@ def bench(workload, m, n, k, kdir=None, launch=None, mode="kernel", warmup=10, r
         kern = _kernel(kdir, launch)
         logical = _logical(workload, m, n, k, launch)
         res = kern.resources(0)
-        geo = kern.launches()[0]
+        geo = kern.launches()[0]["run"]
     else:
         kern = _blas_kernel(workload, m, n, k)
         logical = None
@@ -261,9 +261,10 @@ def bench(workload, m, n, k, kdir=None, launch=None, mode="kernel", warmup=10, r
 
 
 def ptxas_resources(kdir):
-    """Registers, spills and LDS of the selected instantiation from the
-    compiler's resource remarks (python/tforge_gpu.py:155-160 read ptxas -v)."""
-    launch = parse_launch(kdir)
+    """Registers, spills and LDS of the kernel that runs (on 16-byte aligned
+    buffers) from the compiler's resource remarks (python/tforge_gpu.py:155-160
+    read ptxas -v)."""
+    launch = parse_launch(kdir)["launches"][0]["run"]
     table = json.loads((pathlib.Path(__file__).resolve().parent / "kernel_resources.json").read_text())
     rec = table.get(launch["kernel"], {})
     return {"regs": rec.get("vgprs", 0), "agprs": rec.get("agprs", 0), "sgprs": rec.get("sgprs", 0),
