@@ -41,7 +41,7 @@ def _run(workload, m, n, k, options, arrays):
 
 @pytest.mark.parametrize("workload", ["mbr", "matmul"])
 @pytest.mark.parametrize("shape,options", [
-    ((200, 140, 72), "block-tile=16,16 thread-tile=1,1"),                 # direct FMA chain
+    ((200, 140, 72), "block-tile=16,16 thread-tile=1,1"),                 # sequential-k chain (other tiles: test_gpu_direct_edges.py)
     ((256, 256, 128), STAGED.format(128, 128, 8, 4, 32)),                 # 32x32 blocks, bias in LDS
     ((256, 256, 128), STAGED.format(64, 64, 4, 4, 16)),                   # one 32x32 block per wave
     ((256, 256, 128), STAGED.format(64, 64, 2, 2, 64)),                   # 16x16 blocks
@@ -115,7 +115,7 @@ def _same(got, want):
 
 @pytest.mark.parametrize("options", ["block-tile=16,16 thread-tile=1,1", "block-tile=4,256 thread-tile=1,4"])
 @pytest.mark.parametrize("workload", ["relu", "bias_add", "add"])
-@pytest.mark.parametrize("n", [132, 130])   # 16-byte aligned rows (128-bit path) and unaligned ones
+@pytest.mark.parametrize("n", [132, 130])   # rows of whole 128-bit vectors, and not
 def test_special_values_through_element_ops(workload, options, n):
     m = 64
     rng = np.random.default_rng(7)

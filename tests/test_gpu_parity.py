@@ -48,6 +48,8 @@ def assert_bound(workload, ins, out):
 @pytest.mark.parametrize("shape", [(256, 256, 128), (67, 17, 33), (777, 1111, 333), (1, 1, 1), (64, 300, 5)])
 @pytest.mark.parametrize("tt", [(1, 1), (2, 2), (4, 4), (8, 4)])
 def test_direct_bitwise_fma(workload, shape, tt):
+    """Aligned buffers: the chains run on the matrix cores whatever the thread tile
+    (the thread tiles' own kernels: test_gpu_unaligned.py)."""
     m, n, k = shape
     tm, tn = tt
     opts = f"block-tile={16 * tm},{16 * tn} thread-tile={tm},{tn}"
@@ -167,8 +169,8 @@ def test_headline_2048(which):
 @pytest.mark.parametrize("opts", ["block-tile=16,16 thread-tile=1,1", "block-tile=4,256 thread-tile=1,4",
                                   "block-tile=8,512 thread-tile=2,8"])
 def test_elementwise_bit_exact(workload, shape, opts):
-    """Scalar and 128-bit paths (thread tiles 4k wide on aligned rows; ragged
-    and unaligned widths fall back per element) are bit-exact."""
+    """Aligned buffers run the flat kernel whatever the options' tiles: bit-exact at
+    every option string (the tiles' own kernels: test_gpu_unaligned.py)."""
     m, n = shape
     d, launch = tg.compile_kernel(workload, m, n, None, opts, tag="test")
     res, out = tg.check(workload, m, n, None, d, launch)
@@ -178,15 +180,14 @@ def test_elementwise_bit_exact(workload, shape, opts):
 
 @pytest.mark.parametrize("workload", ["relu", "bias_add", "add"])
 @pytest.mark.parametrize("opts,shape", [
-    ("block-tile=16,16 thread-tile=1,1", (37, 512)),     # the reference default, 32-bit path
-    ("block-tile=16,16 thread-tile=2,2", (20, 1024)),    # 2 x 2 per thread, 32-bit path
-    ("block-tile=4,256 thread-tile=1,4", (5, 2048)),     # one 128-bit vector per thread
-    ("block-tile=8,512 thread-tile=2,8", (9, 4096)),     # 4 vectors per thread
+    ("block-tile=16,16 thread-tile=1,1", (37, 512)),     # the reference default
+    ("block-tile=16,16 thread-tile=2,2", (20, 1024)),
+    ("block-tile=4,256 thread-tile=1,4", (5, 2048)),
+    ("block-tile=8,512 thread-tile=2,8", (9, 4096)),
 ])
 def test_elementwise_row_chunks_bit_exact(workload, opts, shape):
     """N a multiple of a workgroup's BM*BN elements and M not a multiple of
-    the block tile (the grid's last row of workgroups is partly past M), on
-    the 32-bit and 128-bit paths, 1 to 4 vectors per thread."""
+    the block tile: the flat kernel does not depend on either."""
     m, n = shape
     d, launch = tg.compile_kernel(workload, m, n, None, opts, tag="test")
     res, out = tg.check(workload, m, n, None, d, launch)
@@ -197,9 +198,8 @@ def test_elementwise_row_chunks_bit_exact(workload, opts, shape):
 @pytest.mark.parametrize("workload", ["relu", "bias_add", "add"])
 def test_elementwise_misaligned_buffers(workload):
     """tf_launch on buffers 4 bytes past a 16-byte boundary (torch views one
-    float into an allocation): the element-op kernel drops to its 32-bit path
-    (and loads the bias in the epilogue) and stays bit-exact; N = 1024 would
-    otherwise take the 128-bit path."""
+    float into an allocation): the options' own element-op kernel runs, one element
+    at a time, and stays bit-exact."""
     import torch
     dev = torch.device("cuda:0")
     m, n = 37, 1024
@@ -443,13 +443,12 @@ def test_masked_edges_equal_pad_path_bits(workload, shape, cfg, extra):
 @pytest.mark.parametrize("shape", [(130, 70, 91), (200, 300, 1010), (97, 130, 313), (65, 66, 109), (64, 64, 96)])
 @pytest.mark.parametrize("cfg", [(64, 64, 4, 4, 16), (128, 64, 8, 4, 16), (128, 128, 8, 8, 64)])
 def test_masked_k_tail_equals_pad_path_bits(workload, shape, cfg):
-    """The end of the K loop of masked kernels: the slab holding row K - 1 is
-    loaded element by element DEPTH slabs before it is stored with the zero
-    fill, after a steady loop of an even number of slabs.  Tile-k 16 (two
-    staging sets): K = 91, 1010, 313, 96, 109 give 6, 64, 20, 6, 7 slabs (an
-    even and an odd count after the steady loop); tile-k 64 (the 128 x 128
-    configuration, one staging set): 5, 16 and 2 slabs.  The pad path's bits
-    and the bound."""
+    """The end of the K loop of masked kernels.  Tile-k 16 (staging spread over the
+    MFMAs): bounded loads, A's columns past K cleared as the last slab is stored; K =
+    91, 1010, 313, 96, 109 give 6, 64, 20, 6, 7 slabs, even and odd counts.  Tile-k 64
+    (the 128 x 128 configuration, block-staged): the slab holding row K - 1 is loaded
+    element by element DEPTH slabs before it is stored with the zero fill; 5, 16 and 2
+    slabs.  The pad path's bits and the bound."""
     m, n, k = shape
     opts = STAGED.format(*cfg)
     ins = o.make_inputs(workload, m, n, k)
@@ -466,8 +465,8 @@ NARROW_SHAPES = [(5, 2, 3), (33, 3, 70), (70, 6, 9), (65, 7, 2), (2, 130, 5), (1
 @pytest.mark.parametrize("shape", NARROW_SHAPES)
 @pytest.mark.parametrize("cfg", [(64, 64, 2, 2, 64), (64, 64, 4, 4, 32)])
 def test_masked_narrow_shapes_equal_pad_path_bits(workload, shape, cfg):
-    """Rows narrower than one 16-byte vector (N < 4: every slab guarded),
-    unaligned rows (N % 4 != 0), K below one k-chunk, on 16x16 and 32x32
+    """Rows narrower than one 16-byte vector (N < 4: block-staged kernels guard
+    every slab), unaligned rows (N % 4 != 0), K below one k-chunk, on 16x16 and 32x32
     MFMA blocks: the pad path's bits and the bound."""
     m, n, k = shape
     opts = STAGED.format(*cfg)
