@@ -1,10 +1,12 @@
 """Maximum sizes: the address arithmetic at the limits of each path.
 
 The unmasked staged kernels address A, B and C with 64-bit offsets, so a
-matrix may exceed 2^31 elements.  Those that stage through buffer loads take a
-32-bit byte offset from each slab's base, which covers BM rows of A and BK rows
-of B while BM * K + BK and BK * N + BN stay below 2^29 elements; past that the
-launch runs the same loop with flat 64-bit loads.  The masked twins use 32-bit
+matrix may exceed 2^31 elements.  Those that stage through buffer loads take
+31-bit byte offsets.  Block-staged ones (two or more waves per SIMD) rebase every
+slab, so BM rows of A and BK rows of B have to fit: BM * K + BK and BK * N + BN below
+2^29 elements.  The spread ones (one wave per SIMD) rebase B every few slabs, so six
+slabs of B have to: 6 * BK * N + BN below 2^29.  Past that the launch runs the same
+loop with flat 64-bit loads.  The masked twins use 32-bit
 offsets and the host rejects problems whose tiles could reach 2^31 elements
 ((M + 256) * K or (K + 64) * (N + 256), runtime select_launches).
 
@@ -73,11 +75,12 @@ def test_masked_kernel_past_its_limit_is_refused():
         _lib.Kernel(tc.gen_mlir("mbr", m, n, k), STAGED.format(64, 64, 4, 4, 32) + " mask-edges=1", "t.mlir")
 
 
-# The spread-staging 128 x 128 kernel (thread-tile 8,8, tile-k 16) on both
-# sides of its buffer-load limit: BM * K + BK (A) or BK * N + BN (B) just below
-# 2^29 elements runs buffer loads whose byte offsets reach 2^31 - 64 KiB or
-# more; one K tile (or one N tile) more runs the flat-load loop.
+# The spread-staging 128 x 128 kernel (thread-tile 8,8, tile-k 16) and the
+# block-staged one (8,4) on both sides of their buffer-load limits: just below 2^29
+# elements they run buffer loads whose byte offsets reach 2^31 - 64 KiB or more; one K
+# tile (or one N tile) more runs the flat-load loop.
 SPREAD_88 = STAGED.format(128, 128, 8, 8, 16)
+BLOCK_84 = STAGED.format(128, 128, 8, 4, 16)
 
 
 @pytest.mark.gpu
@@ -93,4 +96,20 @@ def test_buffer_load_limit_in_b(n):
     """B is 96 x ~2^25 (12 GiB), C 128 x ~2^25 (16 GiB); six K slabs, so the
     slab loop's own loads (slabs 3 to 5) take the path under test."""
     assert (16 * n + 128 < 1 << 29) == (n == 33554304)
-    _exact_case(128, n, 96, SPREAD_88)
+    _exact_case(128, n, 96, BLOCK_84)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [5592320, 5592448, 33554432])
+def test_spread_buffer_load_limit_in_b(n):
+    """The same for six slabs of B; below the limit B is walked two slabs per window."""
+    assert (6 * 16 * n + 128 < 1 << 29) == (n == 5592320)
+    _exact_case(128, n, 144, SPREAD_88)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k", [(5592391, 137), (5592407, 137), (5592407, 5), (6000001, 32)])
+def test_masked_spread_kernel_past_six_slabs_of_b(n, k):
+    """The masked twin's flat-load loop: guarded slab, K tail, edges in M and N."""
+    assert (6 * 16 * n + 64 < 1 << 29) == (n == 5592391)
+    _exact_case(63, n, k, STAGED.format(64, 64, 4, 4, 16) + " mask-edges=1")
