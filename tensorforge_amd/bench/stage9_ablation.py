@@ -1,14 +1,18 @@
 #!/usr/bin/env python3
 """What each optimisation buys for relu(A @ B + bias) on MI355X: an ablation
-ladder from three unfused naive kernels to the autotuned fused kernel.
+ladder from three unfused programs to the autotuned fused kernel.
 
-Rungs (the first five are the reference's, by name and meaning --
+Rungs (the first five are the reference's, by name and options --
 bench/stage9_ablation.py -- so the two tables line up row by row):
 
-  baseline    matmul, bias_add and relu as three direct kernels (16x16 blocks,
-              one output per thread); time = the sum of the three medians,
-              each kernel checked on its own
-  +fusion     one direct kernel with the epilogue fused
+  baseline    matmul, bias_add and relu as three programs with the reference's
+              naive options (16x16 blocks, one output per thread); time = the
+              sum of the three medians, each checked on its own
+  +fusion     one such program with the epilogue fused
+              (Both run what those options run here: the same sequential-k chains on
+              the matrix cores, the element ops as one vector stream.  So they are
+              the cost of a program without options, not of naive code, and the
+              next two rungs, the ablated staged kernels, can be slower.)
   +tiling     the reference's default tiles, 128x64 blocks, 8x4 per thread,
               K step 16, as FP32 MFMA on fragments read from global memory
   +promotion  ... with the A and B slabs staged through LDS

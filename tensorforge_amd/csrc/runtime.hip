@@ -133,16 +133,18 @@ long ceil_div(long a, long b) { return (a + b - 1) / b; }
 // the results are the same bits whichever tile runs.
 //
 // Predicted time = start + rounds * K * cost, rounds = ceil(tiles / 256) (one
-// workgroup per CU each); the tile with the least runs.  Measured on MI355X:
-// cost 5.6-6.0 ns per k for 32x32 tiles, 15.1-16.4 for 64x64, 59-60 for 128x128
-// (masked twins about 1/12 more), start 2.7, 3.4 and 5.7 us.  Both sides of
-// the lines (us, back to back): 32 / 64 at 700^3 11.2 / 16.1, 900^3 22.0 / 20.1,
-// 1100^3 38.5 / 38.8, 64x4096x4096 24.0 / 71.9; 64 / 128 at 1800x1800x500
-// 37.5 / 42.7, 2048^3 126.1 / 125.3, 4096x4096x1024 256.8 / 247.4,
-// 4095x4097x1023 283.0 / 324.6.  With the small tile a K of 2048 or more takes
-// tile-k 64: one workgroup per CU streams its operands, and twice the loads in
-// flight carry it (64x4096x4096 33.0 -> 24.0, 64x2048x2048 12.7 -> 12.1); below
-// that tile-k 32 starts sooner and pads less (700^3 11.2 against 12.2).
+// workgroup per CU each); the tile with the least runs.  Fitted on MI355X: cost
+// 5.6-6.0 ns per k for 32x32 tiles, 15.1-16.4 for 64x64, 59-60 for 128x128 (masked
+// twins about 1/12 more), start 2.7, 3.4 and 5.7 us.  Both sides of the lines
+// (us, back to back, the buffers changing): 32 / 64 at 700^3 11.6 / 16.6, 900^3 21.6 /
+// 20.5, 1100^3 29.3 / 36.9, 64x4096x4096 22.3 / 64.8; 64 / 128 at 1800x1800x500
+// 38.6 / 42.1, 2048^3 124.2 / 125.1, 4096x4096x1024 247.7 / 246.2,
+// 4095x4097x1023 274 / 318.  (The kernels have gained since the fit, the 32x32 tile
+// most where several share a CU: 4.2 ns per k at 1536^3, where the rule takes 64x64,
+// 70.6 us, and 32x32 would take 61.1; 1792x1792x512 35.4 with 128x128, 31.9 with 32x32.)
+// With the small tile a K of 2048 or more takes tile-k 64: one workgroup per CU
+// streams its operands, and twice the loads in flight carry it (64x4096x4096
+// 24.9 -> 22.3, 64x2048x2048 13.7 -> 12.2); below that tile-k 32 pads less.
 const tfk::KernelEntry *seq_entry(long M, long N, long K) {
   struct Tile {
     long edge, cost, start;  // tenths of ns

@@ -30,8 +30,8 @@
 //    The K tail of A is padded with -0.0: -0.0 * +0.0 = -0.0 leaves every
 //    accumulator as it is, a -0.0 included (+0.0 would make it +0.0).  Bound
 //    by the same matrix pipes as the staged kernels; back to back, one thread
-//    per output -> this: 256x256x128 15.2 -> 3.5 us, 777x1111x333 132 -> 11.4,
-//    1000^3 376-471 -> 21.3, 2048^3 3763 -> 125.3 (137 TFLOP/s).
+//    per output -> this: 256x256x128 15.0 -> 3.3 us, 777x1111x333 132.8 -> 10.9,
+//    1000^3 471 -> 20.9, 2048^3 3763 -> 125.4 (137 TFLOP/s).
 //  * Staging (promote=1).  A tile [BM][BK+4 or +8] and B tile [BK][BN+8 or +4] in LDS,
 //    double-buffered, one barrier per slab.  Two register staging sets where
 //    a thread stages few vectors: the global loads of slab t+3 are issued in
@@ -39,10 +39,10 @@
 //    middle of slab t+2), so the LDS writes do not wait on HBM latency under
 //    full-chip load (one set, 1.5 slabs ahead, for the register-heavy
 //    configurations); the slab loop is unrolled by two so buffer and set
-//    indices are compile-time.  The barrier sits before the slab's last chunk so those MFMAs hide the next slab's first LDS reads.  Each
-//    chunk's MFMAs are scheduled around the next chunk's fragment reads in a
-//    measured order.  Row padding makes the b128 fragment reads and the b32
-//    B reads bank-conflict-free.
+//    indices are compile-time.  The barrier sits before the slab's last chunk so
+//    those MFMAs hide the next slab's first LDS reads.  Each chunk's MFMAs are
+//    scheduled around the next chunk's fragment reads in a measured order.  Row
+//    padding makes the b128 fragment reads and the b32 B reads bank-conflict-free.
 //  * Epilogue in registers: bias (staged in LDS during the prologue when the
 //    chain starts with bias_add), IEEE relu, residual add; 128-bit stores.
 //  * vectorize=1: 128-bit global loads and LDS accesses; vectorize=0: 32-bit.
@@ -226,14 +226,15 @@ struct StagedGemm {
   static constexpr int B_ROW_G = SEQ ? 1 : 4, B_ROW_S = SEQ ? 64 / MB : 1;
   static constexpr int A_ELEMS = BM * LDA, B_ELEMS = BK * LDB;
   // Two A and B tile buffers, plus the tile's BN bias values.
-  // Crowded grids (64x64 t4x4 k16, chosen by crowd_entry in runtime.hip).  A slab is
-  // half of each 128-byte line of its A rows, and the plain form's five or six
-  // workgroups per CU keep more lines in flight than outlive the L1 until the next
-  // slab wants the other half: padded to four per CU.  And a branch to the next
-  // instruction before a slab's first LDS write: it empties the wave's instruction
-  // buffer, and waves that meet at their writes drift apart.  (Found by timing: 16
-  // idle cycles there are slower on small grids and no better on large ones, s_sleep
-  // 0 does nothing, waiting for all but the newest load does half of it.)  us, plain /
+  // Crowded grids (64x64 t4x4 k16, chosen by crowd_entry in runtime.hip), padded to
+  // four workgroups per CU: five or six walk more rows and columns of tiles at once
+  // than an XCD's L2 holds, and refetch them (HBM reads, MiB, plain / this form:
+  // 4096x4096x1024 442 / 321, masked 4095x4097x1023 516 / 364; the L1 asks the L2 as
+  // often in both, 17.3 / 17.6 M and 22.6 / 24.1 M requests).  And a branch to the next
+  // instruction before a slab's first LDS write, which empties the wave's instruction
+  // buffer.  Why that helps is not settled.  (Found by timing: 16 idle cycles there are
+  // slower on small grids and no better on large ones, s_sleep 0 does nothing,
+  // waiting for all but the newest load does half of it.)  us, plain /
   // padded / padded with the branch: unmasked 2112x3328x704 92.0 / 82.6 / 82.3,
   // 3008x3008x1008 156.6 / 158.3 / 146.9, 4096x4096x1024 275.9 / 275.8 / 262.7; masked
   // 2600x2900x1200 165.4 / 155.6 / 155.6, 3000x3000x1000 158.7 / 160.0 / 149.0,
@@ -373,7 +374,9 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     constexpr int DEPTH = (G::A_PER + G::B_PER) <= 8 ? 2 : 1;
     VT ra[DEPTH][G::A_PER], rb[DEPTH][G::B_PER];
 
-    // Masked instantiations (MASK = 1).  Rows of A at or past M and columns of B at
+    // Masked instantiations (MASK = 1) that stage in blocks, and those that spread
+    // their staging where six slabs of B pass 2 GiB (the rest use bounded loads,
+    // below).  Rows of A at or past M and columns of B at
     // or past N only reach outputs that are never stored, so a slab that does
     // not hold the last K row loads them from a nearby valid element (row
     // M-1, column N-4) with the same 128-bit loads as the unmasked path.
@@ -567,11 +570,12 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     // rebuilt from k0 every slab took 45 scalar instructions, which with one wave
     // per SIMD do not fit beside an MFMA: masked 1000^3 25.0 us.)  Against
     // flat or per-slab buffer loads with guarded, conditional tails, us back to
-    // back: masked 64x64 t4x4 k16 777x1111x333 10.9 -> 9.9, 1000^3 20.0 -> 18.8,
-    // 4095x4097x1023 274 -> 270; unmasked 32x32 t2x2 k32 512^3 5.34 -> 4.98,
-    // 512x512x2048 12.0 -> 11.2, 64x64 t4x4 k16 1024^3 18.2 -> 17.95; 128x128 t8x8
-    // k16 2048^3 120.5 -> 120.4.  VGPRs of the masked kernels: 99 -> 66 (64x64),
-    // 171 -> 113 (128x128).
+    // back, the buffers changing between launches: masked 64x64 t4x4 k16 777x1111x333
+    // 11.8 -> 10.8, 2100x2100x700 68.8 -> 57.6, masked 128x128 t8x8 k16 2000^3 129.5 ->
+    // 126.7; unmasked 32x32 t2x2 k32 512^3 6.53 -> 5.78, 512x512x2048 17.7 -> 13.6,
+    // 64x64 t4x4 k16 1024^3 22.6 -> 20.0; 128x128 t8x8 k16 2048^3 121.1 -> 121.7 (level
+    // on other boxes), 32x32 at 64^3 2.83 -> 2.97: three slabs are loaded whatever K.
+    // VGPRs of the masked kernels: 99 -> 66 (64x64), 171 -> 113 (128x128).
     __amdgpu_buffer_rsrc_t rsa, rsb;
     SlabOffsets at;  // scalar offsets of the next slab to load
     const int a_step = BK * 4, b_step = BK * (int)ldb * 4;
