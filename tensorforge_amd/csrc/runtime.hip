@@ -174,13 +174,14 @@ const tfk::KernelEntry *seq_entry(long M, long N, long K) {
 }
 
 // The crowded-grid form of staged entry `e` (StagedGemm::CROWD), or null: none, or
-// the grid has no more workgroups than its plain form runs at once, six per CU.
-// Both sides, us, plain / crowded: unmasked 2048x2048x1024 (1024 workgroups) 68.6 /
-// 68.7, 2112x2112x704 (1089) 58.9 / 59.9, 2560x2560x512 (1600) 61.7 / 61.6,
-// 2112x3328x704 (1716) 92.0 / 82.3; masked 2100x2100x700 (1089) 63.1 / 64.9,
-// 2100x3300x700 (1716) 91.7 / 85.9.
+// the grid has no more workgroups than its plain form runs at once, six per CU or,
+// masked, five (its registers).  Both sides, us by workgroups, plain / crowded: unmasked,
+// K = 704, 1088 55.3 / 58.4, 1225 57.2 / 65.0, 1520 72.3 / 71.4, 1584 82.4 / 77.0, 1760
+// 93.8 / 80.8, 2070 101.0 / 97.9, 2600 123.5 / 122.8, 3068 146.7 / 139.0; masked, K = 701,
+// 1088 57.2 / 63.8, 1225 59.6 / 67.7, 1296 68.9 / 68.0, 1360 75.9 / 68.3, 1520 82.6 /
+// 76.1, 1760 89.5 / 84.9, 2070 102.1 / 102.5, 2600 128.9 / 127.6, 3068 153.7 / 145.2.
 const tfk::KernelEntry *crowd_entry(const tfk::KernelEntry &e, dim3 grid) {
-  if ((long)grid.x * grid.y * grid.z <= 6 * 256) return nullptr;
+  if ((long)grid.x * grid.y * grid.z <= (e.masked ? 5 : 6) * 256) return nullptr;
   for (int i = 0; i < tfk::kFormCount; ++i) {
     const tfk::KernelEntry &f = tfk::kFormEntries[i];
     if (f.family == tfk::FAM_STAGED && e.family == f.family && f.bm == e.bm && f.bn == e.bn && f.tm == e.tm &&

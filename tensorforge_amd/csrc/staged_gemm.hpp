@@ -227,10 +227,14 @@ struct StagedGemm {
   static constexpr int A_ELEMS = BM * LDA, B_ELEMS = BK * LDB;
   // Two A and B tile buffers, plus the tile's BN bias values.
   // Crowded grids (64x64 t4x4 k16, chosen by crowd_entry in runtime.hip), padded to
-  // four workgroups per CU: five or six walk more rows and columns of tiles at once
-  // than an XCD's L2 holds, and refetch them (HBM reads, MiB, plain / this form:
-  // 4096x4096x1024 442 / 321, masked 4095x4097x1023 516 / 364; the L1 asks the L2 as
-  // often in both, 17.3 / 17.6 M and 22.6 / 24.1 M requests).  And a branch to the next
+  // four workgroups per CU.  The plain form's six (masked five) start and end together,
+  // and a grid a little larger leaves the rest to run one per CU, with nothing to
+  // overlap its waits; of four, more are left and run together (MFMA busy, plain / this
+  // form: 2112x3328x704 62 / 70%, masked 2100x3300x700 62 / 68%, at the same HBM reads,
+  // 98 / 101 and 101 / 103 MiB).  On grids of several rounds six also walk more rows and
+  // columns of tiles at once than an XCD's L2 holds, and refetch them (HBM reads, MiB:
+  // 4096x4096x1024 464 / 320, masked 4095x4097x1023 528 / 364; the L1 asks the L2 as
+  // often in both, 17.0 / 17.6 M and 22.5 / 24.1 M requests).  And a branch to the next
   // instruction before a slab's first LDS write, which empties the wave's instruction
   // buffer.  Why that helps is not settled.  (Found by timing: 16 idle cycles there are
   // slower on small grids and no better on large ones, s_sleep 0 does nothing,

@@ -1,5 +1,5 @@
 """The 64x64 t4x4 k16 kernels' crowded-grid form (more than six workgroups per CU,
-split-K included) gives the bits of the plain form: the same rows computed in two
+masked five, split-K included) gives the bits of the plain form: the same rows computed in two
 launches of half the workgroups each, below the line."""
 
 import numpy as np
@@ -23,11 +23,12 @@ def _mbr(a, b, bias, opts):
     return out
 
 
-# 1540 workgroups (one row of tiles more than the line's 1536), the line itself
-# and grids that several rounds of workgroups cover; K of one slab to several.
+# 1540 workgroups (one row of tiles more than the line's 1536; masked 1312, the line at
+# 1280), the line itself and grids that several rounds of workgroups cover; K of one slab to several.
 @pytest.mark.parametrize("m,n,extra", [(2240, 2816, ""), (2304, 2816, " split-k=1"), (2240, 2811, " mask-edges=1"),
                                        (2303, 4094, " mask-edges=1"), (1280, 2560, " split-k=2"),
-                                       (1279, 2559, " mask-edges=1 split-k=2"), (2048, 3072, "")])
+                                       (1279, 2559, " mask-edges=1 split-k=2"), (2048, 3072, ""),
+                                       (2047, 2623, " mask-edges=1"), (2047, 2559, " mask-edges=1")])
 @pytest.mark.parametrize("k", [32, 48, 96, 208])
 def test_crowded_form_is_bitwise_the_plain_form(m, n, extra, k):
     import torch

@@ -24,9 +24,13 @@ CASES = [
      "tf_elementwise_flat_uint32_t_true_w8s32", [512, 1, 1], [512, 1, 1]),
     ("add", 16384, 16384, None, "", "tf_elementwise_t1x1", "tf_elementwise_flat_uint32_t_true_w4s4", [262144, 1, 1],
      [256, 1, 1]),
-    # 1536 workgroups and one row of tiles more; split-K ranges count
+    # 1536 workgroups (masked 1280) and one row of tiles more; split-K ranges count
     ("mbr", 2048, 3072, 64, MID, "tf_staged_b64x64_t4x4_k16", "tf_staged_b64x64_t4x4_k16", [48, 32, 1], [16, 16, 1]),
     ("mbr", 2112, 3072, 64, MID, "tf_staged_b64x64_t4x4_k16", "tf_staged_b64x64_t4x4_k16_crowd", [48, 33, 1], [16, 16, 1]),
+    ("mbr", 2047, 2559, 61, MID + " mask-edges=1", "tf_staged_b64x64_t4x4_k16_masked", "tf_staged_b64x64_t4x4_k16_masked",
+     [40, 32, 1], [16, 16, 1]),
+    ("mbr", 2049, 2559, 61, MID + " mask-edges=1", "tf_staged_b64x64_t4x4_k16_masked",
+     "tf_staged_b64x64_t4x4_k16_masked_crowd", [40, 33, 1], [16, 16, 1]),
     ("mbr", 1025, 3000, 64, MID + " mask-edges=1 split-k=2", "tf_staged_b64x64_t4x4_k16_masked",
      "tf_staged_b64x64_t4x4_k16_masked_crowd", [47, 17, 2], [16, 16, 1]),
     ("mbr", 4096, 4096, 64, STAGED.format("64,64", "4,4", 32), "tf_staged_b64x64_t4x4_k32", "tf_staged_b64x64_t4x4_k32",
@@ -43,6 +47,18 @@ def test_run_kernel(workload, m, n, k, options, own, run, grid, block):
     if own == run:
         assert (got["grid"], got["block"], got["lds_bytes"]) == (launch["grid"], launch["block"], launch["lds_bytes"])
     assert got["lds_bytes"] == RES[run]["lds_bytes"]
+
+
+@pytest.mark.parametrize("mask,per_cu", [("", 6), ("_masked", 5)])
+def test_crowded_line_is_what_the_plain_form_runs_at_once(mask, per_cu):
+    """Four waves a workgroup: waves per SIMD = workgroups per CU.  The crowded form
+    takes the first grid past 256 CUs of them (the CASES above)."""
+    assert RES[f"tf_staged_b64x64_t4x4_k16{mask}"]["occupancy_waves_per_simd"] == per_cu
+    assert RES[f"tf_staged_b64x64_t4x4_k16{mask}_crowd"]["occupancy_waves_per_simd"] == 4
+    for gy, crowd in ((per_cu * 8, False), (per_cu * 8 + 1, True)):
+        opts = MID + (" mask-edges=1" if mask else "")
+        run = _lib.Kernel(tc.gen_mlir("mbr", gy * 64, 2048, 64), opts, "t.mlir").launches()[0]["run"]
+        assert run["kernel"] == f"tf_staged_b64x64_t4x4_k16{mask}" + ("_crowd" if crowd else "")
 
 
 def test_compiler_resources_are_the_run_kernels(tmp_path, monkeypatch):
