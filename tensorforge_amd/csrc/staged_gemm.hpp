@@ -578,7 +578,7 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     // 11.8 -> 10.8, 2100x2100x700 68.8 -> 57.6, masked 128x128 t8x8 k16 2000^3 129.5 ->
     // 126.7; unmasked 32x32 t2x2 k32 512^3 6.53 -> 5.78, 512x512x2048 17.7 -> 13.6,
     // 64x64 t4x4 k16 1024^3 22.6 -> 20.0; 128x128 t8x8 k16 2048^3 121.1 -> 121.7 (level
-    // on other boxes), 32x32 at 64^3 2.83 -> 2.97: three slabs are loaded whatever K.
+    // on other boxes).
     // VGPRs of the masked kernels: 99 -> 66 (64x64), 171 -> 113 (128x128).
     __amdgpu_buffer_rsrc_t rsa, rsb;
     SlabOffsets at;  // scalar offsets of the next slab to load
@@ -876,8 +876,13 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     // beside the buffer one spills there, as it does in masked block-staged
     // kernels with 512 threads and tile-k 32 or 64.
     if constexpr (SPREAD) {
-      // (Six slabs of B at least: three in flight, two computed per iteration.)
-      if ((long)BM * lda + BK < kBufElems && 6L * BK * ldb + BN < kBufElems) {
+      // (Six slabs of B at least: three in flight, two computed per iteration.  Of one
+      // or two slabs unmasked kernels load no more than those, below; with three loads
+      // whatever K, us, before them / bounded / as now: 64x64 t4x4 k64 640x64448x64 96.7 /
+      // 113.4 / 98.5, 5184x128x128 5.6 / 6.3 / 5.8, k16 1024x1024x16 3.8 / 4.1 / 3.8, 32x32
+      // t2x2 k32 2048x2048x32 10.3 / 11.8 / 10.1.  Of three on bounded loads are level
+      // or ahead at most sizes.  Masked kernels gain from the first slab on.)
+      if ((MASK || nk >= 3) && (long)BM * lda + BK < kBufElems && 6L * BK * ldb + BN < kBufElems) {
         // Slab t is staged in register set t & 1.
         using Bounded = std::integral_constant<int, 2>;
         using Closing = std::integral_constant<int, 3>;

@@ -67,6 +67,24 @@ def test_nan_stays_in_its_row_and_column(cfg, k):
     assert (np.abs(out[keep] - ref[keep]) <= bound[keep]).all()
 
 
+# Unmasked kernels take bounded loads from three slabs on, masked ones always; the
+# masked problem has one column more, and its other columns are the same bits.
+@pytest.mark.parametrize("cfg", TILES + [(64, 64, 4, 4, 64), (32, 32, 2, 2, 64)])
+@pytest.mark.parametrize("slabs,extra", [(1, ""), (2, ""), (3, ""), (4, ""), (5, ""), (4, " split-k=2"), (5, " split-k=2")])
+def test_few_slabs_unmasked_is_bitwise_masked(cfg, slabs, extra):
+    bm, bn, _, _, bk = cfg
+    m, n, k = 2 * bm, 3 * bn, slabs * bk
+    ins = o.make_inputs("mbr", m, n + 1, k)
+    a, b, bias = (np.ascontiguousarray(v) for v in ins.values())
+    opts = STAGED.format(*cfg) + extra
+    masked = _lib.Kernel(tc.gen_mlir("mbr", m, n + 1, k), opts, "t.mlir")
+    plain = _lib.Kernel(tc.gen_mlir("mbr", m, n, k), opts.replace(" mask-edges=1", ""), "t.mlir")
+    assert not plain.launches()[0]["run"]["kernel"].endswith("_masked")
+    want = _launch(masked, [a, b, bias], m, n + 1)[:, :n]
+    got = _launch(plain, [a, np.ascontiguousarray(b[:, :n]), np.ascontiguousarray(bias[:n])], m, n)
+    assert not np.isnan(got).any() and o.bitwise_diff(got, np.ascontiguousarray(want)) == 0
+
+
 # 2^29 elements of B fit one window; past that the loop rebases its resource, every two
 # slabs at N = 5e6.  Entries in {-1, 0, 1}: exact in any order.
 @pytest.mark.parametrize("shape,mask", [((128, 16384, 40000), 0), ((127, 16381, 40003), 1), ((64, 5000000, 208), 0),
