@@ -876,13 +876,16 @@ staged_gemm_kernel(const float *pA, const float *pB, long plda, long pldb, int p
     // beside the buffer one spills there, as it does in masked block-staged
     // kernels with 512 threads and tile-k 32 or 64.
     if constexpr (SPREAD) {
-      // (Six slabs of B at least: three in flight, two computed per iteration.  Of one
-      // or two slabs unmasked kernels load no more than those, below; with three loads
-      // whatever K, us, before them / bounded / as now: 64x64 t4x4 k64 640x64448x64 96.7 /
-      // 113.4 / 98.5, 5184x128x128 5.6 / 6.3 / 5.8, k16 1024x1024x16 3.8 / 4.1 / 3.8, 32x32
-      // t2x2 k32 2048x2048x32 10.3 / 11.8 / 10.1.  Of three on bounded loads are level
-      // or ahead at most sizes.  Masked kernels gain from the first slab on.)
-      if ((MASK || nk >= 3) && (long)BM * lda + BK < kBufElems && 6L * BK * ldb + BN < kBufElems) {
+      // (Six slabs of B at least: three in flight, two computed per iteration.  Unmasked
+      // kernels of up to four slabs load flat, below: bounded loads set up resources and
+      // load three slabs whatever K.  us, before bounded loads / bounded / flat: one slab,
+      // 64x64 t4x4 k64 640x64448 96.7 / 113.4 / 98.5, 32x32 t2x2 k32 2048^2 10.3 / 11.8 /
+      // 10.1; three, 64x64 t4x4 k16 1024^2 4.36 / 4.65 / 4.49, 32x32 640x1504 5.23 / 5.49 /
+      // 5.23; four, 32x32 2048^2 16.4 / 16.0 / 15.6, 64x64 t4x4 k32 6016x512 11.5 / 11.8 /
+      // 11.5, k16 1024^2 4.65 / 4.93 / 4.79 but 1856x3840 15.4 / 15.3 / 15.7.  With twelve
+      // slabs flat loads are behind: 1024x1024x192 6.7 bounded, 6.9 flat.  Masked kernels
+      // gain from the first slab on.)
+      if ((MASK || nk >= 5) && (long)BM * lda + BK < kBufElems && 6L * BK * ldb + BN < kBufElems) {
         // Slab t is staged in register set t & 1.
         using Bounded = std::integral_constant<int, 2>;
         using Closing = std::integral_constant<int, 3>;

@@ -67,10 +67,11 @@ def test_nan_stays_in_its_row_and_column(cfg, k):
     assert (np.abs(out[keep] - ref[keep]) <= bound[keep]).all()
 
 
-# Unmasked kernels take bounded loads from three slabs on, masked ones always; the
+# Unmasked kernels take bounded loads from five slabs on, masked ones always; the
 # masked problem has one column more, and its other columns are the same bits.
 @pytest.mark.parametrize("cfg", TILES + [(64, 64, 4, 4, 64), (32, 32, 2, 2, 64)])
-@pytest.mark.parametrize("slabs,extra", [(1, ""), (2, ""), (3, ""), (4, ""), (5, ""), (4, " split-k=2"), (5, " split-k=2")])
+@pytest.mark.parametrize("slabs,extra", [(1, ""), (2, ""), (3, ""), (4, ""), (5, ""), (6, ""), (4, " split-k=2"),
+                                         (9, " split-k=2"), (10, " split-k=2")])
 def test_few_slabs_unmasked_is_bitwise_masked(cfg, slabs, extra):
     bm, bn, _, _, bk = cfg
     m, n, k = 2 * bm, 3 * bn, slabs * bk

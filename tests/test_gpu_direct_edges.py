@@ -45,10 +45,10 @@ def _uniform(*shape):
 
 # (tile and tile-k, M x N that the size rule gives it, K)
 ENDS = ([("b32x32_t2x2_k32", s, k) for s in ((32, 32), (33, 65), (1, 3))
-         for k in (1, 3, 31, 32, 33, 36, 63, 64, 65, 95, 96, 97, 127, 128, 129, 161)] +
+         for k in (1, 3, 31, 32, 33, 36, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 161, 192)] +
         [("b32x32_t2x2_k64", s, k) for s in ((32, 32), (33, 65)) for k in (2048, 2049, 2051, 2111, 2112, 2113, 2240)] +
         [("b64x64_t4x4_k16", s, k) for s in ((4096, 4096), (4095, 4093))
-         for k in (7, 15, 16, 17, 20, 31, 32, 33, 47, 48, 49, 63, 64, 65, 81)] +
+         for k in (7, 15, 16, 17, 20, 31, 32, 33, 47, 48, 49, 63, 64, 65, 80, 81, 96)] +
         [("b128x128_t8x8_k16", s, k) for s in ((8192, 8192), (8191, 8190)) for k in (63, 64, 65, 79, 80, 81, 99)])
 
 
